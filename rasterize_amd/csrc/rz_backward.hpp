@@ -81,81 +81,42 @@ __device__ inline bool path_tile(const SceneFineArgs& a, uint32_t q, int TX, int
 __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
   const SceneFineArgs& a = b.f;
   if (a.st->err || a.st->overflow) return;
-  __shared__ TileLDS L;
+  __shared__ TileLDS<kGroup> L;
   const int lane = threadIdx.x;
   const int TX = (int)(blockIdx.x % (uint32_t)a.tiles_x), TY = (int)(blockIdx.x / (uint32_t)a.tiles_x);
-  const int col = lane & 15;
   const uint32_t nrow = a.row_count[TY];
   const uint32_t* row = a.rows + (size_t)TY * a.n_paths;
+  // the lane's pixels in a path's tile slot
+  const int pix = lane_row(lane) * 16 + lane_col(lane);
   rzp::C4 c[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) c[k] = a.bg;
-  // forward sweep
-  for (uint32_t start = 0; start < nrow; start += 64) {
-    const uint32_t j = start + lane;
-    uint32_t pid = 0;
-    bool hit = false;
-    if (j < nrow) {
-      pid = row[j];
-      const int4 r = a.rects[pid];
-      hit = r.x <= TX && TX < r.z;
-    }
-    // a path with zero winding over the tile is skipped (the reverse sweep
-    // writes its zero dL/dW)
-    uint32_t lt = 0, lrb = 0, lre = 0, leb = 0, lee = 0;
-    const bool draw = hit && path_tile(a, pid, TX, TY, &lt, &lrb, &lre, &leb, &lee);
-    uint64_t m = __ballot(draw);
-    while (m) {
-      const int src = __ffsll((unsigned long long)m) - 1;
-      m &= m - 1;
-      const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)pid, src);
-      const PathInfo& P = a.pi[q];
-      const int txl = TX - P.tx0, tyl = TY - P.ty0;
-      const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)lt, src);
-      const uint32_t rb = (uint32_t)__builtin_amdgcn_readlane((int)lrb, src);
-      const uint32_t re = (uint32_t)__builtin_amdgcn_readlane((int)lre, src);
-      const uint32_t eb = (uint32_t)__builtin_amdgcn_readlane((int)leb, src);
-      const uint32_t ee = (uint32_t)__builtin_amdgcn_readlane((int)lee, src);
-      const bool local = rb != re || eb != ee;
-      const int64_t bd = (int64_t)a.bd[t] << rzg::kFixShift;
-      if (local) tile_coverage(L, a.recs, rb, re, a.events, eb, ee, txl, lane);
-      const int xs = txl * 16 - P.g.phx + col;
+  for (int i = 0; i < 4; ++i) c[i] = a.bg;
+  // forward sweep; a path with zero winding over the tile is skipped (the
+  // reverse sweep writes its zero dL/dW)
+  scene_paths(
+      a, L, TX, TY, lane, [](const PathInfo&, auto w) { return (float)w * (1.0f / kFix); },
+      [&](const PathInfo& P, uint32_t, uint32_t t, int xs, int ys, const float* W) {
+        const size_t e = (size_t)t * 256 + pix;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int r = 4 * k + (lane >> 4);
-        int64_t w = bd;
-        if (local) w += tile_local(L, k, lane);
-        const int ys = tyl * 16 - P.g.phy + r;
-        float W = 0.0f;
-        const size_t e = (size_t)t * 256 + (size_t)(r * 16 + col);
-        if (xs >= 0 && xs < P.g.W && ys >= 0 && ys < P.g.H) {
-          if (xs >= P.redge_col) {
-            const int64_t rr = a.redge[P.redge_base + ys];
-            w += xs == P.redge_col ? (int64_t)rint((double)rr * P.redge_w) : rr;
-          }
-          W = (float)w * (1.0f / kFix);
-          const float alpha = alpha_of(P.rule, W);
+        for (int i = 0; i < 4; ++i) {
+          const float alpha = alpha_of(P.rule, W[i]);
           if (alpha >= 1e-6f) {
             // the colour below is needed only where the path is drawn (the
             // reverse sweep tests the same alpha)
-            b.pbuf[e] = c[k];
-            c[k] = rzp::blend_over(c[k], rzp::mul(rzp::paint_at(P.paint, xs, ys), alpha));
+            b.pbuf[e + i] = c[i];
+            c[i] = rzp::blend_over(c[i], rzp::mul(rzp::paint_at(P.paint, xs + i, ys), alpha));
           }
         }
-        b.wbuf[e] = W;
-      }
-      if (local) __syncthreads();
-    }
-  }
+        *(float4*)(b.wbuf + e) = make_float4(W[0], W[1], W[2], W[3]);
+      });
   // reverse sweep
   rzp::C4 g[4];
   float T[4];
-  const int x = TX * 16 + col;
+  const int x = TX * 16 + lane_col(lane), y = TY * 16 + lane_row(lane);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int y = TY * 16 + 4 * k + (lane >> 4);
-    g[k] = (x < a.lw && y < a.lh) ? b.grad_out[(size_t)y * b.grad_stride + x] : rzp::splat(0.0f);
-    T[k] = 1.0f;
+  for (int i = 0; i < 4; ++i) {
+    g[i] = (x + i < a.lw && y < a.lh) ? b.grad_out[(size_t)y * b.grad_stride + x + i] : rzp::splat(0.0f);
+    T[i] = 1.0f;
   }
   const uint32_t nchunks = (nrow + 63) / 64;
   for (uint32_t ci = nchunks; ci-- > 0;) {
@@ -185,12 +146,14 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
     auto prefetch = [&](uint64_t mm) {
       if (!mm) return;
       const int s2 = 63 - __clzll((long long)mm);
-      const size_t base = (size_t)(uint32_t)__builtin_amdgcn_readlane((int)lt, s2) * 256 + lane;
+      const size_t base = (size_t)(uint32_t)__builtin_amdgcn_readlane((int)lt, s2) * 256 + pix;
+      const float4 w = *(const float4*)(b.wbuf + base);
+      nW[0] = w.x;
+      nW[1] = w.y;
+      nW[2] = w.z;
+      nW[3] = w.w;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        nW[k] = b.wbuf[base + 64 * k];
-        nB[k] = b.pbuf[base + 64 * k];
-      }
+      for (int k = 0; k < 4; ++k) nB[k] = b.pbuf[base + k];
     };
     prefetch(m);
     while (m) {
@@ -208,19 +171,18 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
       const PathInfo& P = a.pi[q];
       const int txl = TX - P.tx0, tyl = TY - P.ty0;
       const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)lt, src);
-      const int xs = txl * 16 - P.g.phx + col;
+      const int xs = txl * 16 - P.g.phx + lane_col(lane);
+      const int ys = tyl * 16 - P.g.phy + lane_row(lane);
       rzp::C4 dc = rzp::splat(0.0f);
+      float gWs[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int r = 4 * k + (lane >> 4);
-        const int ys = tyl * 16 - P.g.phy + r;
-        const size_t e = (size_t)t * 256 + (size_t)(r * 16 + col);
         float gW = 0.0f;
-        if (xs >= 0 && xs < P.g.W && ys >= 0 && ys < P.g.H) {
+        if (xs + k >= 0 && xs + k < P.g.W && ys >= 0 && ys < P.g.H) {
           const float W = cW[k];
           const float alpha = alpha_of(P.rule, W);
           if (alpha >= 1e-6f) {
-            const rzp::C4 cp = rzp::paint_at(P.paint, xs, ys);
+            const rzp::C4 cp = rzp::paint_at(P.paint, xs + k, ys);
             const rzp::C4 below = cB[k];
             const float gdot = g[k].r * below.r + g[k].g * below.g + g[k].b * below.b + g[k].a * below.a;
             const rzp::C4 ds = rzp::c4(T[k] * g[k].r, T[k] * g[k].g, T[k] * g[k].b, T[k] * (g[k].a - gdot));
@@ -230,7 +192,7 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
             int i0, i1;
             float w1;
             rzp::C4 mixed;
-            if (b.stop_acc && rzp::gradient_stops_at(P.paint, xs, ys, &i0, &i1, &w1, &mixed)) {
+            if (b.stop_acc && rzp::gradient_stops_at(P.paint, xs + k, ys, &i0, &i1, &w1, &mixed)) {
               // through into_linear and the stops' lerp (GradStops::at)
               rzp::C4 gm = rzp::mul(ds, alpha);
               if (!P.paint.linear_colors) gm = rzp::into_linear_vjp(mixed, gm);
@@ -250,8 +212,9 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
             T[k] *= 1.0f - cp.a * alpha;
           }
         }
-        b.wbuf[e] = gW;
+        gWs[k] = gW;
       }
+      *(float4*)(b.wbuf + (size_t)t * 256 + pix) = make_float4(gWs[0], gWs[1], gWs[2], gWs[3]);
       // dL/dc: reduce over the wave, one atomic per channel
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) {

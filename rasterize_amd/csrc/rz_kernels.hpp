@@ -1447,51 +1447,41 @@ constexpr float kFix = (float)(1 << rzg::kFixShift);
 
 __device__ inline int fix(float v) { return __float2int_rn(v * kFix); }
 
-// Inclusive prefix sum inside each 16-lane DPP row (row_shr:1,2,4,8).
-__device__ inline int row_scan16(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-  return v;
-}
+// The coverage of one tile is accumulated in LDS: 16 rows of kAccStride ints,
+// columns 0..15 the deposits of the pixels, column kRowD the row's share of
+// the V terms (add_v). A stride of 20 keeps four pixels a 16-byte LDS read
+// and puts the same column of the 16 rows into 16 different banks
+// (neighbouring lanes often deposit into neighbouring rows of one steep
+// record).
+constexpr int kAccStride = 20;
+constexpr int kAccInts = 16 * kAccStride;
+constexpr int kRowD = 16;
 
-// Add sign * V(yc) to the per-row base, V(yc)(row) = clamp(yc - row, 0, 1),
-// stored as differences between consecutive rows (prefix-summed later). The
-// difference of row 0 goes to the lane's own sum r0 (added to rowd[0] once
-// per tile by flush_row0: an atomic on one address from many lanes would be
-// serialized lane by lane).
-__device__ inline void add_v(int* rowd, uint32_t& r0, float yc, float sign) {
+// A lane's pixels of a tile: four consecutive ones of row lane_row, from
+// column lane_col. The rows run upwards with the lane, so that the sum over
+// the rows below (lane_windings) is a prefix over lanes.
+__device__ inline int lane_row(int lane) { return 15 - (lane >> 2); }
+__device__ inline int lane_col(int lane) { return (lane & 3) << 2; }
+
+// Add sign * V(yc), V(yc)(row) = clamp(yc - row, 0, 1), stored as differences
+// whose sum over the rows at and below a row is the row's value: at most two
+// rows change.
+__device__ inline void add_v(int* acc, float yc, float sign) {
   if (!(yc > 0.0f)) return;
+  const int one = (int)(sign * kFix);
   if (yc >= 16.0f) {
-    r0 += (uint32_t)(int)(sign * kFix);
+    atomicAdd(&acc[15 * kAccStride + kRowD], one);
     return;
   }
-  int k = (int)yc;
-  float f = yc - (float)k;
-  int one = (int)(sign * kFix), ff = fix(sign * f);
-  if (k == 0) {
-    r0 += (uint32_t)ff;
-  } else {
-    r0 += (uint32_t)one;
-    atomicAdd(&rowd[k], ff - one);
-  }
-  atomicAdd(&rowd[k + 1], -ff);
+  const int k = (int)yc;
+  const int ff = fix(sign * (yc - (float)k));
+  atomicAdd(&acc[k * kAccStride + kRowD], ff);
+  if (k > 0) atomicAdd(&acc[(k - 1) * kAccStride + kRowD], one - ff);
 }
 
-// Add the lanes' row-0 sums to rowd[0] (two's-complement sums, exact in any
-// order). Every lane of the wave takes part.
-__device__ inline void flush_row0(int* rowd, uint32_t r0, int lane) {
-  const uint32_t t = (uint32_t)__builtin_amdgcn_readlane(dpp_add_scan((int)r0), 63);
-  if (lane == 0 && t) atomicAdd(&rowd[0], (int)t);
-}
-
-// The tile's accumulators are rows of kAccStride ints: with 17, the same
-// column of different rows falls in different LDS banks (neighbouring lanes
-// often deposit into neighbouring rows of one steep record).
-constexpr int kAccStride = 17;
+// A deposit of v (in 2^-20 units) into a pixel of the tile.
 __device__ inline void dep(int* acc, int row, int col, float v) {
-  if ((unsigned)col < 16u) atomicAdd(&acc[row * kAccStride + col], fix(v));
+  if ((unsigned)col < 16u) atomicAdd(&acc[row * kAccStride + col], __float2int_rn(v));
 }
 
 // signed_difference_line (src/rasterize.rs:395-469) for the cell records of
@@ -1499,17 +1489,20 @@ __device__ inline void dep(int* acc, int row, int col, float v) {
 // the right and are accounted for by their backdrops.
 //
 // A record crosses one to 16 pixel rows. The records are taken 64 at a time,
-// one per lane (left-edge crossings, direction, slope and row range), and
-// their (record, row) pairs are then dealt out to the lanes 64 at a time, so
-// a record crossing many rows keeps many lanes busy rather than one. A row's
-// x range is computed from the record's start and slope (x0 + dx/dy (y - y0)).
+// one per lane (left-edge crossings, direction, slope and row range). Where
+// none of the 64 crosses more than two rows (curves flatten into lines of
+// about a pixel) each lane deposits its own record's rows; otherwise the
+// (record, row) pairs are dealt out to the lanes 64 at a time, so a record
+// crossing many rows keeps many lanes busy rather than one. A row's x range
+// is computed from the record's start and slope (x0 + dx/dy (y - y0)).
 
-// A record prepared for its row steps, staged in LDS for the wave.
+// A record prepared for its row steps.
 struct RowStage {
-  float x0, y0, y1, dxdy, dir;
-  int ys;   // first row
+  float x0, y0, y1, dxdy;
+  float dir;     // +-2^20: deposits are in 2^-20 units
+  int ys;        // first row
   uint32_t pre;  // first row step of the record among its round's steps
-  int pad;
+  int acc;       // offset of its tile's accumulators
 };
 
 // Deposit the part of a prepared record within pixel row y.
@@ -1549,34 +1542,68 @@ __device__ inline void fine_row(int* acc, const RowStage& R, int y) {
   }
 }
 
-// Records [rb, re) of one tile into the wave's LDS accumulators (the row-0
-// differences into the lane's row0, see add_v). `rs` and `marks` are the
-// wave's 64-entry LDS scratch. Every lane of the wave takes part.
-__device__ inline void tile_records(const float4* recs, uint32_t rb, uint32_t re, int* acc,
-                                    int* rowd, uint32_t& row0, RowStage* rs, int* marks, int lane) {
+// The LDS of one wave's coverage: the accumulators of up to G tiles (2^-20
+// fixed point, int32), and for a tile accumulated in chunks the int64 sums of
+// the lanes' pixels ([i][lane]), which take the place of tiles 1 and 2.
+template <int G>
+struct TileLDS {
+  alignas(16) int acc[G >= 3 ? G : 1][kAccInts];
+  RowStage rs[64];
+  int marks[64];
+  long long w64_own[G >= 3 ? 1 : 4 * 64];
+  __device__ long long* w64() { return G >= 3 ? (long long*)acc[G >= 3 ? 1 : 0] : w64_own; }
+};
+static_assert(2 * kAccInts * sizeof(int) >= 4 * 64 * sizeof(long long), "w64 lies over two tiles");
+
+// The records of up to G tiles, those of tile g at recs[rb[g] + j - pre[g]]
+// for pre[g] <= j < pre[g + 1], into the tiles' accumulators. Every lane of
+// the wave takes part; rb and pre are uniform.
+template <int G>
+__device__ inline void tile_records(const float4* recs, const uint32_t (&rb)[G],
+                                    const uint32_t (&pre)[G + 1], TileLDS<G>& L, int lane) {
+  const uint32_t n = pre[G];
+  auto tile_of = [&](uint32_t j, uint32_t* at) {
+    uint32_t base = rb[0];
+    int g = 0;
+#pragma unroll
+    for (int i = 1; i < G; ++i)
+      if (j >= pre[i]) {
+        g = i;
+        base = rb[i] - pre[i];
+      }
+    *at = base + j;
+    return g;
+  };
   // each round's records are loaded while the previous round is deposited
-  float4 nx = rb + (uint32_t)lane < re ? recs[rb + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
-  for (uint32_t r0 = rb; r0 < re; r0 += 64) {
+  uint32_t at;
+  int ng = tile_of((uint32_t)lane, &at);
+  float4 nx = (uint32_t)lane < n ? recs[at] : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (uint32_t r0 = 0; r0 < n; r0 += 64) {
     const uint32_t i = r0 + (uint32_t)lane;
     int nrows = 0;
     RowStage R{};
     const float4 cur = nx;
-    if (r0 + 64 + (uint32_t)lane < re) nx = recs[r0 + 64 + lane];
-    if (i < re) {
+    R.acc = ng * kAccInts;
+    if (r0 + 64 < n) {
+      ng = tile_of(i + 64, &at);
+      if (i + 64 < n) nx = recs[at];
+    }
+    if (i < n) {
       const float4 r = cur;
       float x0 = r.x, y0 = r.y, x1 = r.z, y1 = r.w;
       // records are clipped to the cell; anything else is skipped rather than
       // allowed to index outside the tile
       if (fabsf(x0) <= 16.0f && fabsf(x1) <= 16.0f && y0 >= 0.0f && y0 <= 16.0f && y1 >= 0.0f &&
           y1 <= 16.0f) {
-        if (signbit(x0)) add_v(rowd, row0, y0, 1.0f);
-        if (signbit(x1)) add_v(rowd, row0, y1, -1.0f);
+        int* acc = L.acc[0] + R.acc;
+        if (signbit(x0)) add_v(acc, y0, 1.0f);
+        if (signbit(x1)) add_v(acc, y1, -1.0f);
         x0 = fabsf(x0);
         x1 = fabsf(x1);
         if (y0 != y1) {
-          float dir = 1.0f;
+          float dir = kFix;
           if (y0 > y1) {
-            dir = -1.0f;
+            dir = -kFix;
             float t = x0; x0 = x1; x1 = t;
             t = y0; y0 = y1; y1 = t;
           }
@@ -1593,32 +1620,28 @@ __device__ inline void tile_records(const float4* recs, uint32_t rb, uint32_t re
         }
       }
     }
+    if (__ballot(nrows > 2) == 0) {
+      int* acc = L.acc[0] + R.acc;
+      if (nrows > 0) fine_row(acc, R, R.ys);
+      if (nrows > 1) fine_row(acc, R, R.ys + 1);
+      continue;
+    }
     uint32_t n_rows;
     R.pre = wave_excl_scan((uint32_t)nrows, lane, &n_rows);
-    if (nrows > 0) rs[lane] = R;
+    wave_lds_sync();  // the previous round's steps have read the records
+    if (nrows > 0) L.rs[lane] = R;
     wave_lds_sync();
     int carry = -1;
     for (uint32_t k0 = 0; k0 < n_rows; k0 += 64) {
-      const int o = task_owner(marks, R.pre, (uint32_t)nrows, k0, lane, &carry);
+      const int o = task_owner(L.marks, R.pre, (uint32_t)nrows, k0, lane, &carry);
       const uint32_t k = k0 + (uint32_t)lane;
       if (k < n_rows) {
-        const RowStage& Q = rs[o];
-        fine_row(acc, Q, Q.ys + (int)(k - Q.pre));
+        const RowStage& Q = L.rs[o];
+        fine_row(L.acc[0] + Q.acc, Q, Q.ys + (int)(k - Q.pre));
       }
     }
-    wave_lds_sync();  // the next round re-stages the records
   }
 }
-
-// The LDS of one tile's coverage (2^-20 fixed point, int32), and the int64
-// per-pixel sums of a tile accumulated in chunks (lane-major: [k][lane]).
-struct TileLDS {
-  int acc[16 * kAccStride];
-  int rowd[18];
-  RowStage rs[64];
-  int marks[64];
-  long long w64[4 * 64];
-};
 
 // The int32 accumulation is exact while a tile's local winding (its records'
 // deposits, their V terms and its band's events) stays inside int32. Per
@@ -1626,70 +1649,103 @@ struct TileLDS {
 // terms of at most 1, each event at most 1, each term with rounding below
 // 2^20 + 9: so |local| <= (3 records + events) (2^20 + 9) < 2^31 below 2000.
 // Larger tiles are accumulated in chunks of at most 600 records and 190
-// events, each chunk's int32 result folded into int64 per pixel.
+// events, each chunk's int32 result folded into int64 per pixel. A backdrop
+// of size b adds b 2^20, so that local winding and backdrop together stay in
+// int32 below 2000 as well (tile_int32).
 constexpr uint32_t kChunkRecords = 600, kChunkEvents = 190;
 __device__ inline bool tile_narrow(uint32_t n_records, uint32_t n_events) {
   return 3ull * n_records + n_events < 2000ull;
 }
+__device__ inline bool tile_int32(uint32_t n_records, uint32_t n_events, int bd) {
+  return bd > -2000 && bd < 2000 &&
+         3ull * n_records + n_events + (unsigned)(bd < 0 ? -bd : bd) < 2000ull;
+}
 
-// One narrow chunk into LDS: records [rb, re), and those of the events
-// [eb, ee) that lie left of tile column `tx` (in the path's grid); then the
-// per-row base prefix. Every lane takes part.
-__device__ inline void chunk_build(TileLDS& L, const float4* recs, uint32_t rb, uint32_t re,
-                                   const int4* events, uint32_t eb, uint32_t ee, int tx, int lane) {
-#pragma unroll
-  for (int k = lane; k < 16 * kAccStride; k += 64) L.acc[k] = 0;
-  if (lane < 18) L.rowd[lane] = 0;
-  __syncthreads();
-  uint32_t r0 = 0;
-  tile_records(recs, rb, re, L.acc, L.rowd, r0, L.rs, L.marks, lane);
+// Clear the accumulators of n tiles.
+__device__ inline void clear_tiles(int* acc, int n, int lane) {
+  int4* a = (int4*)acc;
+  for (int k = lane; k < n * (kAccInts / 4); k += 64) a[k] = make_int4(0, 0, 0, 0);
+}
+
+// The events [eb, ee) of a band that lie left of tile column `tx` (in the
+// path's grid) into one tile's accumulators.
+__device__ inline void tile_events(int* acc, const int4* events, uint32_t eb, uint32_t ee, int tx,
+                                   int lane) {
   for (uint32_t i = eb + lane; i < ee; i += 64) {
     const int4 ev = events[i];
-    if (ev.y < tx) add_v(L.rowd, r0, __int_as_float(ev.z), __int_as_float(ev.w));
+    if (ev.y < tx) add_v(acc, __int_as_float(ev.z), __int_as_float(ev.w));
   }
-  flush_row0(L.rowd, r0, lane);
+}
+
+// The local windings of the lane's four pixels from a tile's accumulators:
+// the pixels' deposits summed along the row (in the lane, then over the four
+// lanes of the row: quad_perm steps) plus the row's V terms (summed over the
+// rows below: the lanes before, in steps of four). Every lane takes part.
+__device__ inline void lane_windings(const int* acc, int lane, int* w) {
+  const int* a = acc + lane_row(lane) * kAccStride;
+  const int4 v = *(const int4*)(a + lane_col(lane));
+  int d = a[kRowD];
+  // row_shr:4, row_shr:8 (the four rows of 16 lanes), row_bcast:15, :31
+  d += __builtin_amdgcn_update_dpp(0, d, 0x114, 0xf, 0xf, false);
+  d += __builtin_amdgcn_update_dpp(0, d, 0x118, 0xf, 0xf, false);
+  // a 16-lane row's total for each of the four lane columns is the same
+  d += __builtin_amdgcn_update_dpp(0, d, 0x142, 0xa, 0xf, false);
+  d += __builtin_amdgcn_update_dpp(0, d, 0x143, 0xc, 0xf, false);
+  const int p1 = v.x + v.y, p2 = p1 + v.z, p3 = p2 + v.w;
+  int t = p3;
+  // quad_perm [0, 0, 1, 2] and [0, 0, 0, 1]: the lane one and two to the left
+  const int m1 = (lane & 3) >= 1 ? -1 : 0, m2 = (lane & 3) >= 2 ? -1 : 0;
+  t += __builtin_amdgcn_update_dpp(0, t, 0x90, 0xf, 0xf, false) & m1;
+  t += __builtin_amdgcn_update_dpp(0, t, 0x40, 0xf, 0xf, false) & m2;
+  const int base = d + t - p3;
+  w[0] = base + v.x;
+  w[1] = base + p1;
+  w[2] = base + p2;
+  w[3] = base + p3;
+}
+
+// One narrow tile (records [rb, re), the band's events [eb, ee)) into
+// accumulator 0. Every lane of the wave takes part.
+template <int G>
+__device__ inline void tile_build(TileLDS<G>& L, const float4* recs, uint32_t rb, uint32_t re,
+                                  const int4* events, uint32_t eb, uint32_t ee, int tx, int lane) {
+  clear_tiles(L.acc[0], 1, lane);
   __syncthreads();
-  // per-row base: prefix of the row differences (lanes 0..15 scan, in place)
-  if (lane < 16) L.rowd[lane] = row_scan16(L.rowd[lane]);
+  uint32_t rbs[G], pre[G + 1];
+  pre[0] = 0;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    rbs[g] = rb;
+    pre[g + 1] = re - rb;
+  }
+  tile_records<G>(recs, rbs, pre, L, lane);
+  tile_events(L.acc[0], events, eb, ee, tx, lane);
   __syncthreads();
 }
 
-// The local winding of one tile (records [rb, re), the band's events [eb, ee))
-// at each lane's four pixels (rows 4k + lane / 16, column lane % 16) into
-// L.w64[k * 64 + lane], which tile_local reads back: the per-pixel sums stay in
-// LDS, not in registers, while records are deposited. A narrow tile is one
-// int32 chunk; a larger one is summed chunk by chunk. Every lane of the wave
-// takes part (the row scans are DPP).
-__device__ inline void tile_coverage(TileLDS& L, const float4* recs, uint32_t rb, uint32_t re,
-                                     const int4* events, uint32_t eb, uint32_t ee, int tx,
-                                     int lane) {
-  const int col = lane & 15;
-  const bool narrow = tile_narrow(re - rb, ee - eb);
-  uint32_t r0 = rb, e0 = eb;
+// A tile of any size, chunk by chunk, into the lanes' int64 sums in L.w64():
+// they stay in LDS, not in registers, while records are deposited (each lane
+// reads back the slots it wrote: no barrier). Every lane takes part.
+template <int G>
+__device__ inline void tile_build_wide(TileLDS<G>& L, const float4* recs, uint32_t rb, uint32_t re,
+                                       const int4* events, uint32_t eb, uint32_t ee, int tx,
+                                       int lane) {
+  long long* w64 = L.w64();
   bool first = true;
   do {
-    const uint32_t r1 = narrow ? re : min(re, r0 + kChunkRecords);
-    const uint32_t e1 = narrow ? ee : min(ee, e0 + kChunkEvents);
-    chunk_build(L, recs, r0, r1, events, e0, e1, tx, lane);
+    const uint32_t r1 = min(re, rb + kChunkRecords), e1 = min(ee, eb + kChunkEvents);
+    tile_build<G>(L, recs, rb, r1, events, eb, e1, tx, lane);
+    int w[4];
+    lane_windings(L.acc[0], lane, w);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int row = 4 * k + (lane >> 4);
-      const long long v = (int32_t)(L.rowd[row] + row_scan16(L.acc[row * kAccStride + col]));
-      L.w64[k * 64 + lane] = first ? v : L.w64[k * 64 + lane] + v;
-    }
+    for (int i = 0; i < 4; ++i)
+      w64[i * 64 + lane] = first ? (long long)w[i] : w64[i * 64 + lane] + w[i];
     first = false;
-    r0 = r1;
-    e0 = e1;
-    // the next chunk clears the LDS; after the last, the barrier keeps the
-    // caller's later uniform global loads scalar (the compiler takes an LDS
-    // store not followed by a barrier as a possible clobber of them)
-    __syncthreads();
-  } while (r0 < re || e0 < ee);
+    rb = r1;
+    eb = e1;
+    __syncthreads();  // the next chunk clears the accumulators
+  } while (rb < re || eb < ee);
 }
-
-// The local winding at the lane's pixel k after tile_coverage (each lane reads
-// the slots it wrote: no barrier).
-__device__ inline int64_t tile_local(const TileLDS& L, int k, int lane) { return L.w64[k * 64 + lane]; }
 
 struct FineArgs {
   const uint32_t* tile_off;
@@ -1707,33 +1763,45 @@ struct FineArgs {
   double redge_w;
 };
 
-// FillRule::alpha_from_winding (src/path.rs:32-46) on a 2^-20 fixed-point winding
-// (the magnitudes converted to f32 are below 2^21, so the 32-bit conversion
-// is exact and equals the 64-bit one)
-template <int RULE>
-__device__ inline float alpha_fix(int64_t w) {
+// FillRule::alpha_from_winding (src/path.rs:32-46) on a 2^-20 fixed-point
+// winding, in int32 or int64 (the magnitudes converted to f32 are at most
+// 2^20: exact)
+template <int RULE, class I>
+__device__ inline float alpha_fix(I w) {
+  constexpr I one = (I)1 << rzg::kFixShift;
   if (RULE == 0) {
-    int64_t a = w < 0 ? -w : w;
-    if (a >= ((int64_t)1 << rzg::kFixShift)) return 1.0f;
-    float v = (float)(int32_t)a * (1.0f / kFix);
+    const I a = min(w < 0 ? -w : w, one);
+    const float v = (float)(int32_t)a * (1.0f / kFix);
     return v < 1e-6f ? 0.0f : v;
   } else {
     // ((w + 1) rem_euclid 2 - 1).abs(): exact on the fixed-point value
-    const int64_t one = (int64_t)1 << rzg::kFixShift;
-    int64_t u = (w + one) & ((one << 1) - 1);
-    int32_t d = (int32_t)(u - one);
+    const int32_t d = (int32_t)(((w + one) & ((one << 1) - 1)) - one);
     return (float)(d < 0 ? -d : d) * (1.0f / kFix);
   }
 }
 
 constexpr int kFineWave = 64;  // one wave per tile
 
-// Per-pixel outputs of the fine stage.
+// Per-pixel outputs of the fine stage: the coverage of `n` pixels from (x, y)
+// to the right (four unless the image ends).
 // Rasterizer::mask: the coverage itself, every pixel of the image.
 struct MaskOut {
   float* out;
   size_t row_stride;  // floats
-  __device__ void put(int x, int y, float alpha) const { out[(size_t)y * row_stride + x] = alpha; }
+  // rows and images start at any float: 16-byte accesses of 4-byte alignment
+  struct __attribute__((packed, aligned(4))) F4 {
+    float v[4];
+  };
+  __device__ void put(int x, int y, int n, const float* alpha) const {
+    float* o = out + (size_t)y * row_stride + x;
+    if (n == 4) {
+      *(F4*)o = F4{{alpha[0], alpha[1], alpha[2], alpha[3]}};
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i < n) o[i] = alpha[i];
+  }
 };
 // Rasterizer::fill (src/rasterize.rs:69-115): pixels that mask_iter yields
 // (alpha >= 1e-6) get dst = dst.blend_over(paint.at(centre).with_alpha(alpha)).
@@ -1741,20 +1809,53 @@ struct FillOut {
   rzp::C4* img;
   size_t row_stride;  // pixels
   rzp::DPaint paint;
-  __device__ void put(int x, int y, float alpha) const {
-    if (!(alpha >= 1e-6f)) return;
-    const rzp::C4 c = rzp::paint_at(paint, x, y);
-    rzp::C4* d = img + (size_t)y * row_stride + x;
-    *d = rzp::blend_over(*d, rzp::mul(c, alpha));
+  __device__ void put(int x, int y, int n, const float* alpha) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i >= n || !(alpha[i] >= 1e-6f)) continue;
+      const rzp::C4 c = rzp::paint_at(paint, x + i, y);
+      rzp::C4* d = img + (size_t)y * row_stride + x + i;
+      *d = rzp::blend_over(*d, rzp::mul(c, alpha[i]));
+    }
   }
 };
 
+// The windings of the lane's pixels of one tile as alphas: the tile's local
+// windings (none without records and events), its backdrop, and at and right
+// of the right-edge column `rcol` (in tile columns) the column's row sum r.
+template <int RULE>
+__device__ inline void tile_alphas(TileLDS<1>& L, bool local, bool narrow, int bd, bool int32,
+                                   int rcol, double redge_w, const long long* redge, bool row_in,
+                                   int lane, float* alpha) {
+  int w[4] = {0, 0, 0, 0};
+  if (local && narrow) lane_windings(L.acc[0], lane, w);
+  if (int32 && rcol > 15) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) alpha[i] = alpha_fix<RULE>(w[i] + bd * (1 << rzg::kFixShift));
+    return;
+  }
+  const int c0 = lane_col(lane);
+  const int64_t r = row_in && c0 + 3 >= rcol ? (int64_t)*redge : 0;
+  const int64_t re = r ? (int64_t)rint((double)r * redge_w) : 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int64_t v = ((int64_t)bd << rzg::kFixShift) +
+                (local && !narrow ? (int64_t)L.w64()[i * 64 + lane] : (int64_t)w[i]);
+    if (c0 + i == rcol) v += re;
+    else if (c0 + i > rcol) v += r;
+    alpha[i] = alpha_fix<RULE>(v);
+  }
+}
+
 // One 16x16 tile per wave (one workgroup per tile, so the hardware balances
 // tiles of very different record counts): records and events into LDS, then
-// four passes of 16-lane DPP row scans (one pixel row per 16 lanes) and
-// coalesced stores.
+// each lane's four pixels and one coalesced store.
+// Bound by VALU issue (the row steps of the records) and LDS round trips; the
+// sums stay in int32 unless the tile needs more, and a lane's four pixels are
+// one 16-byte LDS read and one store: 200k segments at 4096x4096 96 -> 87 us,
+// 16,384 glyphs 378 -> 328 us.
 template <int RULE, class Out>
-__device__ inline void fine_tile(const FineArgs& a, const Out& o, TileLDS& L) {
+__device__ inline void fine_tile(const FineArgs& a, const Out& o, TileLDS<1>& L) {
   const int lane = threadIdx.x;
   const uint32_t tile = blockIdx.x;
   const int tx = (int)(tile % (uint32_t)a.tiles_x), ty = (int)(tile / (uint32_t)a.tiles_x);
@@ -1762,25 +1863,18 @@ __device__ inline void fine_tile(const FineArgs& a, const Out& o, TileLDS& L) {
   const uint32_t eb = a.band_ev_off[ty], ee = a.band_ev_off[ty + 1];
   // a tile with no records and no events of its band has the winding of its
   // backdrop (plus the right-edge column) everywhere: no LDS work
-  const bool local = rb != re || eb != ee;
-  const int64_t bd = (int64_t)a.bd[tile] << rzg::kFixShift;
-  if (local) tile_coverage(L, a.recs, rb, re, a.events, eb, ee, tx, lane);
-  const int col = lane & 15;
-  const int x = tx * 16 + col;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int row = 4 * k + (lane >> 4);
-    int64_t w = bd;
-    if (local) w += tile_local(L, k, lane);
-    const int y = ty * 16 + row;
-    if (x < a.W && y < a.H) {
-      if (x >= a.redge_col) {
-        const int64_t r = a.redge[y];
-        w += x == a.redge_col ? (int64_t)rint((double)r * a.redge_w) : r;
-      }
-      o.put(x, y, alpha_fix<RULE>(w));
-    }
+  const bool local = rb != re || eb != ee, narrow = tile_narrow(re - rb, ee - eb);
+  const int bd = a.bd[tile];
+  if (local) {
+    if (narrow) tile_build<1>(L, a.recs, rb, re, a.events, eb, ee, tx, lane);
+    else tile_build_wide<1>(L, a.recs, rb, re, a.events, eb, ee, tx, lane);
   }
+  const int x = tx * 16 + lane_col(lane), y = ty * 16 + lane_row(lane);
+  const int rcol = a.redge_col == INT32_MAX ? INT32_MAX : a.redge_col - tx * 16;
+  float alpha[4];
+  tile_alphas<RULE>(L, local, narrow, bd, tile_int32(re - rb, ee - eb, bd), rcol, a.redge_w,
+                    a.redge + y, y < a.H, lane, alpha);
+  if (x < a.W && y < a.H) o.put(x, y, min(4, a.W - x), alpha);
 }
 
 // The status merge (one thread of block 0) comes after the tile's work: a
@@ -1788,7 +1882,7 @@ __device__ inline void fine_tile(const FineArgs& a, const Out& o, TileLDS& L) {
 // tile's uniform data with scalar loads.
 template <int RULE, class Out>
 __global__ __launch_bounds__(kFineWave) void k_fine(FineArgs a, Out o) {
-  __shared__ TileLDS L;
+  __shared__ TileLDS<1> L;
   if (!(a.st->err || a.st->overflow)) fine_tile<RULE>(a, o, L);
   if (blockIdx.x == 0 && threadIdx.x == 0) merge_status(a.st, a.acc);
 }
