@@ -145,7 +145,7 @@ struct rz_ctx {
   DBuf stops;     // gradient stops of the current fill: f64 positions, then C4 colours
   // batched scene render
   DBuf line_path;  // path of each line
-  DBuf bw_w, bw_p, bw_tr;  // scene backward: per-(path, tile) winding / dL/dW, colour below, transform partials
+  DBuf bw_w, bw_d, bw_tr;  // scene backward: per-(path, tile) winding / dL/dW, <dL/d layer, colour below>, transform partials
   DBuf bw_stops;           // scene backward: dL/d(stop as read) per stop of the scene
   DBuf sc_order;           // queued scene fine: tile order, queue head, per-tile path counts
   int n_cus = 256;         // compute units of the device
@@ -1683,7 +1683,7 @@ rz_status enqueue_scene_backward(rz_ctx* ctx, const rz_dscene* s, const rz_trans
   RZ_TRY(enqueue_scene_batched(ctx, s, tr, view, bg, mode, flatness, nullptr, 0));
   const size_t entries = ctx->sc_cap_t;
   RZ_TRY(ensure(ctx, ctx->bw_w, entries * 256 * sizeof(float)));
-  RZ_TRY(ensure(ctx, ctx->bw_p, entries * 256 * sizeof(rzp::C4)));
+  RZ_TRY(ensure(ctx, ctx->bw_d, entries * 256 * sizeof(float)));
   const uint32_t ct = ctx->sc_cap_t, cb = ctx->sc_cap_b;
   const size_t sw = rzk::kStatusWords;
   uint32_t* meta = (uint32_t*)ctx->meta.p;
@@ -1714,7 +1714,7 @@ rz_status enqueue_scene_backward(rz_ctx* ctx, const rz_dscene* s, const rz_trans
   bt.grad_out = (const rzp::C4*)grad_out;
   bt.grad_stride = grad_stride;
   bt.wbuf = (float*)ctx->bw_w.p;
-  bt.pbuf = (rzp::C4*)ctx->bw_p.p;
+  bt.dbuf = (float*)ctx->bw_d.p;
   bt.grad_colors = grad_colors;
   bt.stop_acc = nullptr;
   bt.stop_base = s->stop_col_dev;
@@ -2759,7 +2759,7 @@ rz_status rz_ctx_destroy(rz_ctx* ctx) {
   DBuf* bufs[] = {&ctx->meta,      &ctx->tile_off,  &ctx->ev_off,    &ctx->sums,
                   &ctx->recs,      &ctx->events,    &ctx->out,       &ctx->lines,
                   &ctx->counts,    &ctx->stops,     &ctx->line_path,
-                  &ctx->bw_w,      &ctx->bw_p,      &ctx->bw_tr,     &ctx->bw_stops,
+                  &ctx->bw_w,      &ctx->bw_d,      &ctx->bw_tr,     &ctx->bw_stops,
                   &ctx->sc_order,
                   &ctx->sc_pi,     &ctx->sc_counts,
                   &ctx->sc_rects,  &ctx->sc_rows,   &ctx->sc_rowcnt, &ctx->list_buf,
