@@ -1421,6 +1421,7 @@ rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transf
   b.redge = redge;
   b.st = st;
   rzg::BinGrid g0{};
+  g0.mode = mode;  // the paths' grids are in pi
   const rzk::GapArgs ga{d->view, x, s->slot_path};
   RZ_TRY(enqueue_bin_count<true>(ctx, lb, g0, pi, ga, bin_fill, &b, !fused));
   if (fused)
@@ -1606,6 +1607,7 @@ rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, dou
   b.redge = redge;
   b.st = st;
   rzg::BinGrid g0{};
+  g0.mode = mode;  // the paths' grids are in pi
   const rzk::GapArgs ga{d->view, x, s->slot_path};
   RZ_TRY(enqueue_bin_count<true>(ctx, lb, g0, pi, ga, bin_fill, &b, !fused));
   if (fused)

@@ -651,6 +651,37 @@ RZ_HD bool tile_record(Pt s, Pt e, double r0, int tx, const BinGrid& g, Rec* out
   return true;
 }
 
+// A piece that stays within one band and one tile column, without a crossing
+// of the band's bottom edge: what the three steps above would make of it is at
+// most one record, and its ends are the piece's own (no intersection is
+// computed). Returns false when the piece needs the steps; else *tile is the
+// record's tile, or -1 when it has none.
+RZ_HD bool single_tile(Pt a, Pt b, const BinGrid& g, int* tile, Rec* out) {
+  int t0, t1;
+  *tile = -1;
+  if (!piece_bands(a, b, g, &t0, &t1) || t1 < t0) return true;
+  if (t0 != t1) return false;
+  const double r0 = (double)(t0 * kTile - g.phy);
+  const double rb = fmin(r0 + (double)kTile, (double)g.H);
+  if (!(fmin(a.y, b.y) >= r0) || !(fmax(a.y, b.y) <= rb)) return false;
+  const double xlo = fmin(a.x, b.x), xhi = fmax(a.x, b.x);
+  const int tx = tile_col(xlo, g);
+  if (tx != tile_col(xhi, g)) return false;
+  const double c0 = (double)(tx * kTile - g.phx);
+  if (tx == 0) {
+    if (xhi <= 0.0) return true;  // in tile 0's left region
+    if (xlo <= 0.0) return false;
+  }
+  if (!(xlo >= c0) || !(xhi <= c0 + (double)kTile)) return false;
+  if (a.y == b.y) return true;
+  out->x0 = (float)(a.x - c0);
+  out->y0 = (float)(a.y - r0);
+  out->x1 = (float)(b.x - c0);
+  out->y1 = (float)(b.y - r0);
+  *tile = t0 * g.tiles_x + tx;
+  return true;
+}
+
 // Enumerate the records and band-boundary crossings of one effective piece
 // a -> b, band by band and left to right.
 //   rec(tile_index, Rec)        -- one cell record
