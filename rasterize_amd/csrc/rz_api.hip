@@ -1095,6 +1095,7 @@ struct rz_dscene {
   // interpolated in), their colours as given, and their index among the
   // scene's given stops (paths in order, each paint's stops as given)
   uint32_t n_stops = 0, n_user_stops = 0;
+  bool long_gradients = false;        // a gradient for the general evaluation (rzk::long_gradient)
   rzp::C4* stop_col_dev = nullptr;
   rzp::C4* stop_lin_dev = nullptr;
   int32_t* stop_user_dev = nullptr;   // -1: a gradient's default stop
@@ -1228,6 +1229,7 @@ rz_status scene_upload_impl(rz_ctx* ctx, const rz_path* const* paths, const rz_p
     for (int k = 0; k < 6; ++k) S.paint_tr[k] = paint_i.tr[k];
     S.paint = pp.p;
     stop_first[i] = stop_pos.size();
+    s->long_gradients = s->long_gradients || rzk::long_gradient(pp.pos.data(), pp.pos.size());
     stop_pos.insert(stop_pos.end(), pp.pos.begin(), pp.pos.end());
     stop_col.insert(stop_col.end(), pp.col.begin(), pp.col.end());
     stop_lin.insert(stop_lin.end(), pp.lin.begin(), pp.lin.end());
@@ -1478,9 +1480,16 @@ rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transf
     }
     const int waves = ctx->cur.scene_waves;
 #define RZ_SCENE_FINE(W, Q)                                                                \
-  RZ_LAUNCH_LDS(ctx, "k_scene_fine", (rzk::k_scene_fine<W, Q>), fgrid, dim3(64), ctx->cur.fine_lds, \
-                a, queue)
-    if (queue) {
+  RZ_LAUNCH_LDS(ctx, "k_scene_fine", (rzk::k_scene_fine<W, Q, false>), fgrid, dim3(64),             \
+                ctx->cur.fine_lds, a, queue)
+    if (s->long_gradients) {
+      if (queue)
+        RZ_LAUNCH_LDS(ctx, "k_scene_fine", (rzk::k_scene_fine<1, true, true>), fgrid, dim3(64),
+                      ctx->cur.fine_lds, a, queue);
+      else
+        RZ_LAUNCH_LDS(ctx, "k_scene_fine", (rzk::k_scene_fine<1, false, true>), fgrid, dim3(64),
+                      ctx->cur.fine_lds, a, queue);
+    } else if (queue) {
       if (waves == 8) RZ_SCENE_FINE(8, true);
       else if (waves == 1) RZ_SCENE_FINE(1, true);
       else RZ_SCENE_FINE(6, true);

@@ -123,16 +123,18 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
   // forward sweep; a path with zero winding over the tile is skipped (the
   // reverse sweep writes its zero dL/dW)
   scene_paths(
-      a, L, TX, TY, lane, [](const PathInfo&, auto w) { return (float)w * (1.0f / kFix); },
-      [&](const PathInfo& P, uint32_t, uint32_t t, int xs, int ys, const float* W) {
+      a, L, TX, TY, lane, [](int, auto w) { return (float)w * (1.0f / kFix); },
+      [&](const rzp::DPaint* paint, int rule, uint32_t, uint32_t t, int xs, int ys, bool,
+          const float* W) {
+        const rzp::DPaint p = load_const(paint);
         const size_t e = (size_t)t * 256 + pix;
         *(float4*)(b.wbuf + e) = make_float4(W[0], W[1], W[2], W[3]);
         *(float4*)(b.dbuf + e) = make_float4(D[0], D[1], D[2], D[3]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float alpha = alpha_of(P.rule, W[i]);
+          const float alpha = alpha_of(rule, W[i]);
           if (alpha >= 1e-6f) {
-            const rzp::C4 s = rzp::mul(rzp::paint_at(P.paint, xs + i, ys), alpha);
+            const rzp::C4 s = rzp::mul(rzp::paint_at(p, xs + i, ys), alpha);
             D[i] = (g[i].r * s.r + g[i].g * s.g + g[i].b * s.b + g[i].a * s.a) + D[i] * (1.0f - s.a);
           }
         }
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
       const float cW[4] = {nW.x, nW.y, nW.z, nW.w}, cD[4] = {nD.x, nD.y, nD.z, nD.w};
       prefetch(m);
       const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)pid, src);
-      const PathInfo& P = a.pi[q];
+      const PathInfo P = load_const(a.pi + q);
       const int txl = TX - P.tx0, tyl = TY - P.ty0;
       const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)lt, src);
       const int xs = txl * 16 - P.g.phx + lane_col(lane);

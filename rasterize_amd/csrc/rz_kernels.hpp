@@ -75,6 +75,22 @@ struct Xform {
   double m[6];
 };
 
+// *p for a uniform p to data that no kernel running now writes (tables made by
+// earlier kernels): through the constant address space, so that it is a scalar
+// load whatever the kernel has stored to LDS or memory before.
+template <class T>
+__device__ inline T load_const(const T* p) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  using Word = const __attribute__((address_space(4))) uint32_t;
+  Word* q = (Word*)(uintptr_t)p;
+  uint32_t w[sizeof(T) / 4];
+#pragma unroll
+  for (size_t i = 0; i < sizeof(T) / 4; ++i) w[i] = q[i];
+  T r;
+  __builtin_memcpy(&r, w, sizeof(T));
+  return r;
+}
+
 // One path of a batched scene as the device sees it in one render: its
 // transform into its sub-view (align * tr, src/scene.rs:425-429), the
 // sub-view's binning grid (phased onto the canvas tile grid), the offsets of

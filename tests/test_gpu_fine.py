@@ -80,3 +80,40 @@ def test_mask_rows_of_any_width(w, h, pad):
         d = np.abs(rows[:, :w] - ref)
         assert d.max() <= MAX_ABS and d.mean() <= MEAN_ABS
         assert got[0] == -1.0 and (rows[:, w:] == -1.0).all() and (got[1 + stride * h:] == -1.0).all()
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 64, 65])
+@pytest.mark.parametrize("spread", [rz.GradSpread.Pad, rz.GradSpread.Repeat, rz.GradSpread.Reflect])
+def test_gradient_stops(n, spread):
+    """Gradients of few and many stops (65: beyond the wave's lanes), stops at
+    equal positions, every spread, linear and sRGB interpolation, focal
+    circles inside, on and outside the outer one (no root: transparent).
+    Colours are f32 through the same formulas: 2e-5, of pixels whose position
+    does not sit on a stop boundary (a jump between equal positions)."""
+    w, h = 50, 35
+    rng = np.random.default_rng(10 * n + spread)
+    pos = np.sort(rng.uniform(0.0, 1.0, n))
+    if n >= 5:
+        pos[2] = pos[1]
+    stops = []
+    for p in pos:
+        a = rng.uniform(0.2, 1.0)
+        stops.append((float(p), LinColor(*(a * rng.uniform(0, 1, 3)), a)))
+    common = dict(spread=spread, tr=Transform.new_rotate(0.3).pre_scale(1.1, 0.9))
+    paints = [
+        rz.GradLinear(stops, linear_colors=False, start=(5.0, 3.0), end=(38.0, 30.0), **common),
+        rz.GradLinear(stops, linear_colors=True, start=(30.0, 3.0), end=(12.0, 9.0), **common),
+        rz.GradRadial(stops, center=(25.0, 16.0), radius=14.0, **common),
+        rz.GradRadial(stops, center=(25.0, 16.0), radius=14.0, fcenter=(20.0, 12.0), fradius=2.0, **common),
+        rz.GradRadial(stops, center=(30.0, 16.0), radius=6.0, fcenter=(14.0, 12.0), fradius=3.0, **common),
+    ]
+    view = (0.0, 0.0, float(w), float(h))
+    for k, paint in enumerate(paints):
+        fl = [(rect(-2.0, 1.5, 44.25, 33.0), paint, FillRule.NonZero),
+              (PathBuilder().move_to((20.0, 18.0)).circle(13.0).build(), paint, FillRule.NonZero)]
+        got = Scene(Scene.GROUP, children=[Scene.fill(*f) for f in fl]).render(
+            SignedDifferenceRasterizer(), I, view, (0.2, 0.3, 0.4, 1.0))
+        ref, _ = O.scene_render([(p, c.abi(), r) for p, c, r in fl], I, view, (0.2, 0.3, 0.4, 1.0))
+        d = np.abs(got.image.astype(np.float64) - ref).max(2)
+        print(f"{n} stops, spread {spread}, paint {k}: max|d|={d.max():.3e}", flush=True)
+        assert np.sort(d.ravel())[-4] <= 2e-5, (n, spread, k)  # at most three pixels on a boundary
