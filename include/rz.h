@@ -463,8 +463,9 @@ rz_status rz_mask_atlas(rz_ctx* ctx, const rz_path* const* paths, const rz_atlas
  * default 0): KB of extra LDS per wave of the flatten, the count pass and the
  * fine stage (fewer waves per SIMD). RZ_PARAM_SCATTER_WAVES (8..18, default
  * 15): the scatter's grid holds at most 2^value waves. RZ_PARAM_SCENE_WAVES
- * (1, 6 or 8, default 6): the batched scene's fine kernel built for that many
- * waves per SIMD (1: registers unbounded). RZ_PARAM_SCENE_QUEUE (0 or 1,
+ * (1, 6 or 8, default 6): the register budget of the batched scene's fine
+ * kernel (1: unbounded; 6: 96 VGPRs, for the five waves per SIMD its LDS
+ * allows; 8: 80 VGPRs). RZ_PARAM_SCENE_QUEUE (0 or 1,
  * default 0): the batched scene's fine stage as a persistent grid taking
  * canvas tiles from a device queue, the tiles covered by the most paths
  * first. RZ_PARAM_FUSED (0 or 1, default 0): flatten and the binning's

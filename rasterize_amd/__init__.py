@@ -528,8 +528,7 @@ class LinColor(tuple):
     def abi(self):
         p = _abi.rz_paint()
         p.kind = _abi.RZ_PAINT_SOLID
-        for i in range(4):
-            p.color[i] = self[i]
+        p.color[:] = self
         return p
 
 
@@ -798,6 +797,12 @@ def png_bytes(image, ctx=None):
     return bytes(buf)
 
 
+def _path_pointers(abi_paths):
+    """A C array of pointers to the given rz_path structs (which must outlive it)."""
+    a = (C.c_void_p * max(len(abi_paths), 1))(*[C.addressof(p) for p in abi_paths])
+    return C.cast(a, C.POINTER(C.POINTER(_abi.rz_path)))
+
+
 class Layer:
     """Rendered layer (src/scene.rs:463-520): `image` (H, W, 4) float32
     premultiplied linear RGBA whose pixel (0, 0) is at (x, y)."""
@@ -918,7 +923,7 @@ class Scene:
         fl = self.fills()
         n = len(fl)
         keep = [f[0].abi() for f in fl]
-        paths = (C.POINTER(_abi.rz_path) * max(n, 1))(*[C.pointer(p) for p in keep])
+        paths = _path_pointers(keep)
         pk = [f[1].abi() for f in fl]
         paints = (_abi.rz_paint * max(n, 1))(*pk)
         rules = (C.c_int32 * max(n, 1))(*[f[2] for f in fl])
@@ -994,7 +999,7 @@ class Scene:
             ps, qs, nodes, children, root = self.node_arrays()
             keep = [p.abi() for p in ps]
             pk = [q.abi() for q in qs]
-            paths = (C.POINTER(_abi.rz_path) * max(len(ps), 1))(*[C.pointer(p) for p in keep])
+            paths = _path_pointers(keep)
             paints = (_abi.rz_paint * max(len(qs), 1))(*pk)
             na = (_abi.rz_scene_node * len(nodes))(*nodes)
             ca = (C.c_uint32 * max(len(children), 1))(*children)
@@ -1441,7 +1446,7 @@ def mask_atlas(paths, slots, atlas, fill_rule=FillRule.NonZero, flatness=DEFAULT
         raise TypeError("atlas must be a contiguous 2D float32 array")
     n = len(paths)
     keep = [p.abi() for p in paths]
-    parr = (C.POINTER(_abi.rz_path) * max(n, 1))(*[C.pointer(p) for p in keep])
+    parr = _path_pointers(keep)
     sarr = (_abi.rz_atlas_slot * max(n, 1))(*slots)
     ctx.check(lib().rz_mask_atlas(ctx.h, parr, sarr, n, flatness, int(fill_rule), edge_mode,
                                   atlas.ctypes.data_as(C.POINTER(C.c_float)), atlas.shape[1],
@@ -1457,7 +1462,7 @@ class DeviceGlyphs:
         self.ctx = ctx or default_context()
         n = len(paths)
         keep = [p.abi() for p in paths]
-        parr = (C.POINTER(_abi.rz_path) * max(n, 1))(*[C.pointer(p) for p in keep])
+        parr = _path_pointers(keep)
         h = C.c_void_p()
         self.ctx.check(lib().rz_scene_upload(self.ctx.h, parr, None, None, n, C.byref(h)))
         self.h = h

@@ -154,6 +154,14 @@ struct rz_ctx {
   DBuf list_buf;  // binning: record list (records, tiles) and event list
   DBuf wave_lines;  // per flatten wave: its lines' first index and count
   DBuf atlas_tiles;  // per atlas tile: what the fine stage needs (AtlasTile)
+  // device memory of one blocking call's paths, scenes and layers (TempScope):
+  // blocks handed out front to back, kept for the next call
+  struct TempBlock {
+    char* p;
+    size_t cap, at;
+  };
+  std::vector<TempBlock> temp;
+  bool temp_open = false;
   DBuf sk_work, sk_out;  // rz_path_stroke: input path and work arrays, output path
   uint32_t rec_cap = 0, ev_cap = 0;
   uint32_t part_cap = 0;  // overflow record-list entries per part
@@ -462,17 +470,77 @@ rz_status validate_path(rz_ctx* ctx, const rz_path* p) {
   return RZ_OK;
 }
 
-template <typename T>
-rz_status upload_array(rz_ctx* ctx, rz_dpath* d, const std::vector<T>& v, const T** out) {
-  size_t bytes = std::max<size_t>(1, v.size()) * sizeof(T);
+// Device memory that lives as long as the resident object it belongs to
+// (recorded in `allocs`), or, inside a TempScope, until the blocking call
+// returns.
+constexpr size_t kTempKeep = (size_t)256 << 20;  // bytes kept between blocking calls at most
+rz_status dev_alloc(rz_ctx* ctx, std::vector<void*>& allocs, size_t bytes, void** out) {
+  bytes = (std::max<size_t>(bytes, 16) + 255) & ~(size_t)255;
+  if (ctx->temp_open)
+    for (auto& b : ctx->temp)
+      if (b.cap - b.at >= bytes) {
+        *out = b.p + b.at;
+        b.at += bytes;
+        return RZ_OK;
+      }
+  const size_t want = ctx->temp_open ? std::max<size_t>(bytes, (size_t)4 << 20) : bytes;
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = hipMalloc(&p, want);
   if (e != hipSuccess) return fail(ctx, RZ_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-  d->allocs.push_back(p);
-  if (!v.empty()) RZ_HIP(ctx, hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
-  *out = (const T*)p;
+  if (ctx->temp_open) ctx->temp.push_back({(char*)p, want, bytes});
+  else allocs.push_back(p);
+  *out = p;
   return RZ_OK;
 }
+
+// A blocking call's device memory: while one is open, dev_alloc takes from
+// the context's blocks instead of allocating for every array of every path
+// (1024 circles through rz_render: 8,200 allocations and as many frees, 42 ms
+// of a 46 ms call). Its end waits for the stream, so nothing in flight reads
+// the blocks when the next call takes them; what exceeds kTempKeep is freed.
+struct TempScope {
+  rz_ctx* ctx;
+  bool mine;
+  explicit TempScope(rz_ctx* c) : ctx(c), mine(!c->temp_open) { c->temp_open = true; }
+  ~TempScope() {
+    if (!mine) return;
+    (void)hipStreamSynchronize(ctx->stream);
+    ctx->temp_open = false;
+    size_t kept = 0, n = 0;
+    for (auto& b : ctx->temp) {
+      b.at = 0;
+      if (kept + b.cap > kTempKeep) {
+        (void)hipFree(b.p);
+      } else {
+        kept += b.cap;
+        ctx->temp[n++] = b;
+      }
+    }
+    ctx->temp.resize(n);
+  }
+};
+
+// Arrays packed on the host for one device block and one copy; `put` returns
+// an array's offset.
+struct Pack {
+  std::vector<char> h;
+  size_t put(const void* src, size_t bytes) {
+    const size_t at = (h.size() + 15) & ~(size_t)15;
+    h.resize(at + std::max<size_t>(bytes, 1));
+    if (bytes) std::memcpy(h.data() + at, src, bytes);
+    return at;
+  }
+  template <typename T>
+  size_t put(const std::vector<T>& v) {
+    return put(v.data(), v.size() * sizeof(T));
+  }
+  // Copies to device block `base` (of h.size() bytes) and waits.
+  rz_status copy(rz_ctx* ctx, void* base) const {
+    RZ_HIP(ctx, hipMemcpyAsync(base, h.data(), h.size(), hipMemcpyHostToDevice, ctx->stream));
+    RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return RZ_OK;
+  }
+};
 
 void dpath_release(rz_dpath* d) {
   for (void* p : d->allocs) (void)hipFree(p);
@@ -487,14 +555,15 @@ void dpath_release(rz_dpath* d) {
 // closing line); `order` groups slots by kind so a block never mixes the
 // line, quad and cubic code paths.
 // ---------------------------------------------------------------------------
-static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out) {
-  RZ_TRY(validate_path(ctx, p));
-  rz_dpath* d = new rz_dpath();
+// The slot tables are made on the host (path_pack) and go with the path's
+// arrays into one block; path_place then points the view at them.
+struct PathAt {
+  size_t pts, kinds, pt_off, slot_item, slot_flags, close_pts, order, gap_slots;
+};
+
+static PathAt path_pack(const rz_path* p, rz_dpath* d, Pack& pk) {
   const uint32_t ns = p->n_segments, nsub = p->n_subpaths;
   const uint32_t npts = ns ? p->point_offsets[ns] : 0;
-  std::vector<double> pts(p->points, p->points + 2 * (size_t)npts);
-  std::vector<uint8_t> kinds(p->kinds, p->kinds + ns);
-  std::vector<uint32_t> pt_off(p->point_offsets, p->point_offsets + ns);
   const uint32_t nslots = ns + nsub;
   std::vector<uint32_t> slot_item(nslots);
   std::vector<uint8_t> slot_flags(nslots, 0);
@@ -554,20 +623,16 @@ static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out)
     nb[kind] = blocks_for(cnt);
     order.resize(before + (size_t)nb[kind] * rzk::kBlock, ~0u);
   }
+  PathAt at;
+  at.pts = pk.put(p->points, 16 * (size_t)npts);
+  at.kinds = pk.put(p->kinds, ns);
+  at.pt_off = pk.put(p->point_offsets, 4 * (size_t)ns);
+  at.slot_item = pk.put(slot_item);
+  at.slot_flags = pk.put(slot_flags);
+  at.close_pts = pk.put(close_pts);
+  at.order = pk.put(order);
+  at.gap_slots = pk.put(gap_slots);
   rzk::DPath& v = d->view;
-  rz_status st;
-  if ((st = upload_array(ctx, d, pts, &v.pts)) != RZ_OK ||
-      (st = upload_array(ctx, d, kinds, &v.kinds)) != RZ_OK ||
-      (st = upload_array(ctx, d, pt_off, &v.pt_off)) != RZ_OK ||
-      (st = upload_array(ctx, d, slot_item, &v.slot_item)) != RZ_OK ||
-      (st = upload_array(ctx, d, slot_flags, &v.slot_flags)) != RZ_OK ||
-      (st = upload_array(ctx, d, close_pts, &v.close_pts)) != RZ_OK ||
-      (st = upload_array(ctx, d, order, &v.order)) != RZ_OK ||
-      (st = upload_array(ctx, d, gap_slots, &v.gap_slots)) != RZ_OK) {
-    dpath_release(d);
-    delete d;
-    return st;
-  }
   v.n_slots = nslots;
   v.n_gaps = (uint32_t)gap_slots.size();
   v.blocks_line = nb[0];
@@ -575,17 +640,40 @@ static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out)
   v.blocks_cubic = nb[2];
   d->n_order = (uint32_t)order.size();
   d->n_slots = nslots;
-  hipError_t e = hipStreamSynchronize(ctx->stream);
-  if (e != hipSuccess) {
-    dpath_release(d);
-    delete d;
-    return fail(ctx, RZ_E_HIP, std::string("upload: ") + hipGetErrorString(e));
-  }
   const rzh::Tr ident = {{1.0, 0.0, 0.0, 0.0, 1.0, 0.0}};
   d->has_bbox = rzh::path_bbox(p, ident, &d->bbox);
   SplitSum sum;
   split_sum(p, ident.m, &sum);
   d->est = sum.est();
+  return at;
+}
+
+static void path_place(rz_dpath* d, const PathAt& at, const char* base) {
+  rzk::DPath& v = d->view;
+  v.pts = (const double*)(base + at.pts);
+  v.kinds = (const uint8_t*)(base + at.kinds);
+  v.pt_off = (const uint32_t*)(base + at.pt_off);
+  v.slot_item = (const uint32_t*)(base + at.slot_item);
+  v.slot_flags = (const uint8_t*)(base + at.slot_flags);
+  v.close_pts = (const double*)(base + at.close_pts);
+  v.order = (const uint32_t*)(base + at.order);
+  v.gap_slots = (const uint32_t*)(base + at.gap_slots);
+}
+
+static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out) {
+  RZ_TRY(validate_path(ctx, p));
+  rz_dpath* d = new rz_dpath();
+  Pack pk;
+  const PathAt at = path_pack(p, d, pk);
+  void* base = nullptr;
+  rz_status st = dev_alloc(ctx, d->allocs, pk.h.size(), &base);
+  if (st == RZ_OK) st = pk.copy(ctx, base);
+  if (st != RZ_OK) {
+    dpath_release(d);
+    delete d;
+    return st;
+  }
+  path_place(d, at, (const char*)base);
   *out = d;
   return RZ_OK;
 }
@@ -1083,7 +1171,11 @@ struct rz_dscene {
   uint64_t serial = g_serial.fetch_add(1);  // renewed by rz_atlas_set
   uint32_t n = 0;
   rz_dpath* all = nullptr;             // every path's segments, for the batched form
-  std::vector<rz_dpath*> per;          // one resident path each, for the plain form
+  // one resident path each, for the plain form (made by its first render, in
+  // one block)
+  mutable std::mutex per_mu;
+  mutable std::vector<rz_dpath*> per;
+  mutable std::vector<void*> per_allocs;
   std::vector<void*> allocs;           // ScenePath table, slot -> path map, stops
   const rzk::ScenePath* sp = nullptr;
   rzk::ScenePath* sp_mut = nullptr;
@@ -1103,23 +1195,30 @@ struct rz_dscene {
   // glyph atlas placement (rz_atlas_set): device slots and slice totals
   rzk::AtlasSlot* atlas_slots = nullptr;
   uint32_t* atlas_tile_glyph = nullptr;  // glyph of each atlas tile
+  std::vector<void*> atlas_allocs;
   SplitEst atlas_est;                    // line estimate under the slots' transforms
   uint32_t atlas_tiles = 0, atlas_bands = 0, atlas_rows = 0;
   bool atlas_ready = false;
-  // host copies of the paths, for Path::bbox(tr) in the plain form
-  std::vector<std::vector<uint8_t>> kinds;
-  std::vector<std::vector<uint32_t>> offs, subs;
-  std::vector<std::vector<double>> pts;
-  std::vector<std::vector<uint8_t>> closed;
+  // host copies of the paths, one after the other: for Path::bbox(tr) and the
+  // resident paths of the plain form, and the atlas's line estimate
+  struct HostRange {
+    size_t seg, off, pt, sub, closed;
+    uint32_t n_segments, n_subpaths;
+  };
+  std::vector<HostRange> host;
+  std::vector<uint8_t> kinds, closed;
+  std::vector<uint32_t> offs, subs;
+  std::vector<double> pts;
   rz_path host_path(uint32_t i) const {
+    const HostRange& r = host[i];
     rz_path p;
-    p.n_segments = (uint32_t)kinds[i].size();
-    p.n_subpaths = subs[i].empty() ? 0 : (uint32_t)subs[i].size() - 1;
-    p.kinds = kinds[i].data();
-    p.point_offsets = offs[i].data();
-    p.points = pts[i].data();
-    p.subpaths = subs[i].data();
-    p.closed = closed[i].data();
+    p.n_segments = r.n_segments;
+    p.n_subpaths = r.n_subpaths;
+    p.kinds = kinds.data() + r.seg;
+    p.point_offsets = offs.data() + r.off;
+    p.points = pts.data() + r.pt;
+    p.subpaths = subs.data() + r.sub;
+    p.closed = closed.data() + r.closed;
     return p;
   }
 };
@@ -1136,12 +1235,14 @@ void scene_release(rz_dscene* s) {
     delete d;
   }
   for (void* p : s->allocs) (void)hipFree(p);
-  if (s->atlas_slots) (void)hipFree(s->atlas_slots);
+  for (void* p : s->per_allocs) (void)hipFree(p);
+  for (void* p : s->atlas_allocs) (void)hipFree(p);
   s->atlas_slots = nullptr;
-  if (s->atlas_tile_glyph) (void)hipFree(s->atlas_tile_glyph);
   s->atlas_tile_glyph = nullptr;
   s->per.clear();
   s->allocs.clear();
+  s->per_allocs.clear();
+  s->atlas_allocs.clear();
   s->all = nullptr;
 }
 
@@ -1197,11 +1298,9 @@ rz_status scene_upload_impl(rz_ctx* ctx, const rz_path* const* paths, const rz_p
     const rz_paint& paint_i = paints ? paints[i] : solid;
     const uint32_t seg0 = (uint32_t)kinds.size(), pt0 = (uint32_t)(pts.size() / 2);
     const uint32_t ns = p->n_segments, nsub = p->n_subpaths, npts = ns ? p->point_offsets[ns] : 0;
-    s->kinds.emplace_back(p->kinds, p->kinds + ns);
-    s->offs.emplace_back(p->point_offsets, p->point_offsets + (ns ? ns + 1 : 0));
-    s->pts.emplace_back(p->points, p->points + 2 * (size_t)npts);
-    s->subs.emplace_back(p->subpaths, p->subpaths + (nsub ? nsub + 1 : 0));
-    s->closed.emplace_back(p->closed, p->closed + nsub);
+    s->host.push_back({kinds.size(), s->offs.size(), pts.size(), s->subs.size(), closed.size(), ns, nsub});
+    if (ns) s->offs.insert(s->offs.end(), p->point_offsets, p->point_offsets + ns + 1);
+    if (nsub) s->subs.insert(s->subs.end(), p->subpaths, p->subpaths + nsub + 1);
     for (uint32_t k = 0; k < ns; ++k) {
       kinds.push_back(p->kinds[k]);
       offs.push_back(pt0 + p->point_offsets[k + 1]);
@@ -1238,9 +1337,6 @@ rz_status scene_upload_impl(rz_ctx* ctx, const rz_path* const* paths, const rz_p
       stop_flag.push_back(pp.p.linear_colors ? 1 : 0);
     }
     if (paint_i.kind != RZ_PAINT_SOLID) user_stops += paint_i.n_stops;
-    rz_dpath* d = nullptr;
-    RZ_TRY(path_upload_impl(ctx, p, &d));
-    s->per.push_back(d);
   }
   if (kinds.empty()) offs.clear();
   rz_path all;
@@ -1253,41 +1349,34 @@ rz_status scene_upload_impl(rz_ctx* ctx, const rz_path* const* paths, const rz_p
   all.closed = closed.data();
   RZ_TRY(path_upload_impl(ctx, &all, &s->all));
   // stops, then the ScenePath table pointing into them
-  auto up = [&](const void* src, size_t bytes, void** dst) -> rz_status {
-    void* p = nullptr;
-    hipError_t e = hipMalloc(&p, std::max<size_t>(bytes, 16));
-    if (e != hipSuccess) return fail(ctx, RZ_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-    s->allocs.push_back(p);
-    if (bytes) RZ_HIP(ctx, hipMemcpy(p, src, bytes, hipMemcpyHostToDevice));
-    *dst = p;
-    return RZ_OK;
-  };
-  void *dpos = nullptr, *dcol = nullptr, *dsp = nullptr, *dslot = nullptr, *dsubs = nullptr;
-  RZ_TRY(up(stop_pos.data(), stop_pos.size() * sizeof(double), &dpos));
-  RZ_TRY(up(stop_col.data(), stop_col.size() * sizeof(rzp::C4), &dcol));
-  void *dlin = nullptr, *duser = nullptr, *dflag = nullptr;
-  RZ_TRY(up(stop_lin.data(), stop_lin.size() * sizeof(rzp::C4), &dlin));
-  RZ_TRY(up(stop_user.data(), stop_user.size() * sizeof(int32_t), &duser));
-  RZ_TRY(up(stop_flag.data(), stop_flag.size(), &dflag));
+  Pack pk;
+  const size_t o_pos = pk.put(stop_pos), o_col = pk.put(stop_col), o_lin = pk.put(stop_lin);
+  const size_t o_user = pk.put(stop_user), o_flag = pk.put(stop_flag);
+  const size_t o_slot = pk.put(slot_path), o_subs = pk.put(subs), o_sp = pk.put(s->host_sp);
+  void* block = nullptr;
+  RZ_TRY(dev_alloc(ctx, s->allocs, pk.h.size(), &block));
+  char* base = (char*)block;
   s->n_stops = (uint32_t)stop_col.size();
   s->n_user_stops = user_stops;
-  s->stop_col_dev = (rzp::C4*)dcol;
-  s->stop_lin_dev = (rzp::C4*)dlin;
-  s->stop_user_dev = (int32_t*)duser;
-  s->stop_flag_dev = (uint8_t*)dflag;
+  s->stop_col_dev = (rzp::C4*)(base + o_col);
+  s->stop_lin_dev = (rzp::C4*)(base + o_lin);
+  s->stop_user_dev = (int32_t*)(base + o_user);
+  s->stop_flag_dev = (uint8_t*)(base + o_flag);
   for (size_t i = 0; i < n; ++i) {
     rzk::ScenePath& S = s->host_sp[i];
-    S.paint.stop_pos = (const double*)dpos + stop_first[i];
-    S.paint.stop_col = (const rzp::C4*)dcol + stop_first[i];
+    S.paint.stop_pos = (const double*)(base + o_pos) + stop_first[i];
+    S.paint.stop_col = (const rzp::C4*)(base + o_col) + stop_first[i];
   }
-  RZ_TRY(up(s->host_sp.data(), n * sizeof(rzk::ScenePath), &dsp));
-  RZ_TRY(up(slot_path.data(), slot_path.size() * sizeof(uint32_t), &dslot));
-  RZ_TRY(up(subs.data(), subs.size() * sizeof(uint32_t), &dsubs));
-  s->sp = (const rzk::ScenePath*)dsp;
-  s->sp_mut = (rzk::ScenePath*)dsp;
-  s->slot_path = (const uint32_t*)dslot;
-  s->subpaths = (const uint32_t*)dsubs;
+  if (n) std::memcpy(pk.h.data() + o_sp, s->host_sp.data(), n * sizeof(rzk::ScenePath));
+  RZ_TRY(pk.copy(ctx, base));
+  s->sp = (const rzk::ScenePath*)(base + o_sp);
+  s->sp_mut = (rzk::ScenePath*)(base + o_sp);
+  s->slot_path = (const uint32_t*)(base + o_slot);
+  s->subpaths = (const uint32_t*)(base + o_subs);
   s->n_points = (uint32_t)(pts.size() / 2);
+  s->kinds = std::move(kinds);
+  s->pts = std::move(pts);
+  s->closed = std::move(closed);
   guard.keep = true;
   *out = s;
   return RZ_OK;
@@ -1506,6 +1595,31 @@ rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transf
   return check_launch(ctx, "scene pass 1");
 }
 
+// The plain form's resident paths, all in one block. Scenes are drawn batched
+// unless the caller asks for the plain form, so its first render makes them.
+rz_status ensure_per(rz_ctx* ctx, const rz_dscene* s) {
+  std::lock_guard<std::mutex> lk(s->per_mu);
+  if (!s->per.empty() || s->n == 0) return RZ_OK;
+  std::vector<rz_dpath*> per(s->n);
+  std::vector<PathAt> at(s->n);
+  Pack pk;
+  for (uint32_t i = 0; i < s->n; ++i) {
+    const rz_path hp = s->host_path(i);
+    per[i] = new rz_dpath();
+    at[i] = path_pack(&hp, per[i], pk);
+  }
+  void* base = nullptr;
+  rz_status st = dev_alloc(ctx, s->per_allocs, pk.h.size(), &base);
+  if (st == RZ_OK) st = pk.copy(ctx, base);
+  if (st != RZ_OK) {
+    for (rz_dpath* d : per) delete d;
+    return st;
+  }
+  for (uint32_t i = 0; i < s->n; ++i) path_place(per[i], at[i], (const char*)base);
+  s->per = std::move(per);
+  return RZ_OK;
+}
+
 // The plain form: Pipeline::render_rec's Fill arm (src/scene.rs:410-430) run
 // path by path, each through the single-path pipeline into its sub-view.
 rz_status enqueue_scene_plain(rz_ctx* ctx, const rz_dscene* s, const rz_transform& tr,
@@ -1514,6 +1628,7 @@ rz_status enqueue_scene_plain(rz_ctx* ctx, const rz_dscene* s, const rz_transfor
   int lx, ly, lw, lh;
   layer_of(view, &lx, &ly, &lw, &lh);
   if (lw == 0 || lh == 0) return RZ_OK;
+  RZ_TRY(ensure_per(ctx, s));
   RZ_LAUNCH(ctx, "k_fill_rgba", rzk::k_fill_rgba, dim3(1024), dim3(256), d_out, lw, lh, row_stride, bg);
   // each path's run merges its status into the context's (enqueue_fine)
   const rzh::Tr T = rzh::tr_of(tr.m);
@@ -1816,24 +1931,20 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
     const uint64_t end = i + 1 < s->n ? v[i + 1].tile_base : t;
     for (uint64_t k = v[i].tile_base; k < end; ++k) tile_glyph[k] = i;
   }
-  if (s->atlas_slots || s->atlas_tile_glyph) {
+  if (!s->atlas_allocs.empty()) {
     RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (s->atlas_slots) RZ_HIP(ctx, hipFree(s->atlas_slots));
-    if (s->atlas_tile_glyph) RZ_HIP(ctx, hipFree(s->atlas_tile_glyph));
-    s->atlas_slots = nullptr;
-    s->atlas_tile_glyph = nullptr;
+    for (void* p : s->atlas_allocs) RZ_HIP(ctx, hipFree(p));
+    s->atlas_allocs.clear();
   }
-  void* p = nullptr;
-  hipError_t e = hipMalloc(&p, std::max<size_t>(v.size(), 1) * sizeof(rzk::AtlasSlot));
-  if (e != hipSuccess) return fail(ctx, RZ_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-  s->atlas_slots = (rzk::AtlasSlot*)p;
-  if (!v.empty()) RZ_HIP(ctx, hipMemcpy(p, v.data(), v.size() * sizeof(rzk::AtlasSlot), hipMemcpyHostToDevice));
-  void* q = nullptr;
-  e = hipMalloc(&q, std::max<size_t>(tile_glyph.size(), 1) * sizeof(uint32_t));
-  if (e != hipSuccess) return fail(ctx, RZ_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-  s->atlas_tile_glyph = (uint32_t*)q;
-  if (!tile_glyph.empty())
-    RZ_HIP(ctx, hipMemcpy(q, tile_glyph.data(), tile_glyph.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  s->atlas_slots = nullptr;
+  s->atlas_tile_glyph = nullptr;
+  Pack pk;
+  const size_t o_slots = pk.put(v), o_glyph = pk.put(tile_glyph);
+  void* base = nullptr;
+  RZ_TRY(dev_alloc(ctx, s->atlas_allocs, pk.h.size(), &base));
+  RZ_TRY(pk.copy(ctx, base));
+  s->atlas_slots = (rzk::AtlasSlot*)((char*)base + o_slots);
+  s->atlas_tile_glyph = (uint32_t*)((char*)base + o_glyph);
   s->atlas_tiles = (uint32_t)t;
   s->atlas_bands = (uint32_t)b;
   s->atlas_rows = (uint32_t)r;
@@ -2122,14 +2233,13 @@ struct TreeRender {
   const rz_paint* paints;
   int mode;
   double flatness;
-  std::vector<void*> allocs;            // layers and masks, freed at the end
+  std::vector<void*> allocs;            // none: the call's TempScope holds layers and masks
   std::vector<rz_dscene*> scenes;       // batches
   std::vector<rz_dpath*> dpaths;        // clip paths
   std::vector<int> batch;               // fills waiting for their layer
 
   ~TreeRender() {
     (void)hipStreamSynchronize(ctx->stream);
-    for (void* p : allocs) (void)hipFree(p);
     for (rz_dscene* s : scenes) {
       scene_release(s);
       delete s;
@@ -2139,12 +2249,7 @@ struct TreeRender {
       delete d;
     }
   }
-  rz_status alloc(size_t bytes, void** p) {
-    hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));
-    if (e != hipSuccess) return fail(ctx, RZ_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-    allocs.push_back(*p);
-    return RZ_OK;
-  }
+  rz_status alloc(size_t bytes, void** p) { return dev_alloc(ctx, allocs, bytes, p); }
   rz_status new_layer(const rzh::BBox& b, rzp::C4 fill, DLayer* L) {
     const double v[4] = {b.mn.x, b.mn.y, b.mx.x, b.mx.y};
     layer_of(v, &L->x, &L->y, &L->w, &L->h);
@@ -2777,6 +2882,7 @@ rz_status rz_ctx_destroy(rz_ctx* ctx) {
                   &ctx->wave_lines, &ctx->atlas_tiles};
   drop_graphs(ctx);
   for (DBuf* b : bufs) free_buf(*b);
+  for (auto& b : ctx->temp) (void)hipFree(b.p);
   for (auto& r : ctx->pending) {
     (void)hipEventDestroy(r.a);
     (void)hipEventDestroy(r.b);
@@ -2830,6 +2936,7 @@ rz_status rz_flatten(rz_ctx* ctx, const rz_path* path, rz_transform tr, double f
                      double* lines, size_t cap, size_t* n_lines) {
   if (!ctx || !n_lines) return RZ_E_ARG;
   if (!(flatness > 0.0)) return fail(ctx, RZ_E_ARG, "flatness must be > 0");
+  TempScope scope(ctx);
   rz_dpath* d = nullptr;
   RZ_TRY(path_upload_impl(ctx, path, &d));
   struct Guard {
@@ -3188,6 +3295,7 @@ rz_status rz_fill(rz_ctx* ctx, const rz_path* path, rz_transform tr, double flat
   if (!paint) return fail(ctx, RZ_E_ARG, "paint is NULL");
   const size_t last = shape.start + (H - 1) * shape.row_stride + (W - 1) * shape.col_stride;
   if (4 * last + 4 > rgba_len) return fail(ctx, RZ_E_ARG, "shape exceeds data");
+  TempScope scope(ctx);
   rz_dpath* d = nullptr;
   RZ_TRY(path_upload_impl(ctx, path, &d));
   struct Guard {
@@ -3229,6 +3337,7 @@ rz_status rz_mask_f32(rz_ctx* ctx, const rz_path* path, rz_transform tr, double 
   if (row_stride < width) return fail(ctx, RZ_E_ARG, "row_stride < width");
   if (width == 0 || height == 0) return RZ_OK;
   if (!out) return fail(ctx, RZ_E_ARG, "out is NULL");
+  TempScope scope(ctx);
   rz_dpath* d = nullptr;
   RZ_TRY(path_upload_impl(ctx, path, &d));
   const size_t bytes = height * row_stride * sizeof(float);
@@ -3270,6 +3379,7 @@ rz_status rz_bin(rz_ctx* ctx, const rz_path* path, rz_transform tr, double flatn
     if (n_events) *n_events = 0;
     return RZ_OK;
   }
+  TempScope scope(ctx);
   rz_dpath* d = nullptr;
   RZ_TRY(path_upload_impl(ctx, path, &d));
   struct Guard {
@@ -3404,6 +3514,7 @@ rz_status rz_render(rz_ctx* ctx, const rz_path* const* paths, const rz_paint* pa
   layer_xywh[3] = lh;
   const size_t px = (size_t)lw * lh;
   if (!rgba || cap_px < px) return RZ_OK;
+  TempScope scope(ctx);
   rz_dscene* s = nullptr;
   RZ_TRY(scene_upload_impl(ctx, paths, paints, fill_rules, n, &s));
   struct Guard {
@@ -3485,6 +3596,7 @@ rz_status rz_render_tree(rz_ctx* ctx, const rz_path* const* paths, size_t n_path
   if (!rgba || cap_px < (size_t)lw * lh || !lw || !lh) return RZ_OK;
   const rzp::C4 c = bg ? rzp::c4(bg[0], bg[1], bg[2], bg[3]) : rzp::splat(0.0f);
   rz_status st = RZ_OK;
+  TempScope scope(ctx);
   for (int attempt = 0; attempt < kRuns; ++attempt) {
     TreeRender R{ctx, &tb, paints, edge_mode, flatness, {}, {}, {}, {}};
     DLayer L;
@@ -3532,6 +3644,7 @@ rz_status rz_mask_atlas(rz_ctx* ctx, const rz_path* const* paths, const rz_atlas
     if ((size_t)slots[i].x + slots[i].width > atlas_width ||
         (size_t)slots[i].y + slots[i].height > atlas_height)
       return fail(ctx, RZ_E_ARG, "glyph slot outside the atlas");
+  TempScope scope(ctx);
   rz_dscene* s = nullptr;
   RZ_TRY(scene_upload_impl(ctx, paths, nullptr, nullptr, n, &s));
   struct Guard {
