@@ -19,6 +19,7 @@
 #include "rz_kernels.hpp"
 #include "rz_scene.hpp"
 #include "rz_backward.hpp"
+#include "rz_direct.hpp"
 #include "rz_encode.hpp"
 #include "rz_tree.hpp"
 #include "rz_stroke_kernels.hpp"
@@ -1199,6 +1200,18 @@ struct rz_dscene {
   SplitEst atlas_est;                    // line estimate under the slots' transforms
   uint32_t atlas_tiles = 0, atlas_bands = 0, atlas_rows = 0;
   bool atlas_ready = false;
+  // glyphs masked by k_atlas_direct: their indices by size class (device),
+  // and what flattening them at a call's threshold needs
+  struct DirectClass {
+    uint32_t first, count;
+    size_t lds;
+  };
+  std::vector<DirectClass> direct;
+  uint32_t n_direct = 0, n_binned = 0;   // glyphs with pixels: direct, and the others
+  const uint32_t* direct_list = nullptr;
+  const uint32_t* direct_slots = nullptr;  // [n + 1] first flatten slot of each glyph
+  double direct_bound = 0.0, direct_coord = 0.0;  // largest flatness bound and coordinate
+  bool points_updated = false;           // the device's points are not the host's any more
   // host copies of the paths, one after the other: for Path::bbox(tr) and the
   // resident paths of the plain form, and the atlas's line estimate
   struct HostRange {
@@ -1667,6 +1680,39 @@ rz_status enqueue_scene_plain(rz_ctx* ctx, const rz_dscene* s, const rz_transfor
   return RZ_OK;
 }
 
+// The glyphs of k_atlas_direct. Few glyphs go in one launch with the LDS of
+// the largest (two workgroups a CU hold them all at once); more in a launch per
+// size class, so that small glyphs are not held to the largest one's occupancy.
+rz_status enqueue_atlas_direct(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, double fl,
+                               float* d_atlas, size_t row_stride, rzk::Status* st) {
+  rzk::DirectArgs a;
+  a.p = s->all->view;
+  a.slots = s->atlas_slots;
+  a.slot_begin = s->direct_slots;
+  a.fl = fl;
+  a.mode = mode;
+  a.out = d_atlas;
+  a.row_stride = row_stride;
+  a.st = st;
+  auto launch = [&](uint32_t first, uint32_t count, size_t lds) {
+    a.list = s->direct_list + first;
+    if (rule == RZ_NONZERO)
+      RZ_LAUNCH_LDS(ctx, "k_atlas_direct<0>", rzk::k_atlas_direct<0>, dim3(count),
+                    dim3(rzk::kDirectBlock), lds, a);
+    else
+      RZ_LAUNCH_LDS(ctx, "k_atlas_direct<1>", rzk::k_atlas_direct<1>, dim3(count),
+                    dim3(rzk::kDirectBlock), lds, a);
+  };
+  if (s->n_direct <= 2 * (uint32_t)ctx->n_cus) {
+    size_t lds = 0;
+    for (const auto& c : s->direct) lds = std::max(lds, c.lds);
+    launch(0, s->n_direct, lds);
+  } else {
+    for (const auto& c : s->direct) launch(c.first, c.count, c.lds);
+  }
+  return check_launch(ctx, "k_atlas_direct");
+}
+
 // Glyph atlas: every path of the set masked into its own atlas view, in one
 // pipeline (flatten and binning in their batched form, one wave per glyph tile).
 rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, double flatness,
@@ -1674,6 +1720,21 @@ rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, dou
   const uint32_t n = s->n;
   if (n == 0 || s->atlas_tiles == 0) return RZ_OK;
   select_params(ctx, atlas_tune_key(s, flatness, mode));
+  const double fl = 16.0 * flatness * flatness;
+  // small glyphs in one workgroup each; ActiveEdgeRasterizer's left edge
+  // (rzg::ae_chain) needs the pipeline, and points replaced on the device may
+  // be outside the bounds made from the host's
+  const bool direct = s->n_direct && mode != RZ_EDGE_NONE && !s->points_updated &&
+                      rzk::direct_ok(s->direct_bound, s->direct_coord, fl);
+  if (direct && s->n_binned == 0) {
+    RZ_TRY(ensure(ctx, ctx->meta, rzk::kStatusWords * 4));
+    RZ_LAUNCH(ctx, "k_fill_u32", rzk::k_fill_u32, dim3(1), dim3(64), (uint32_t*)ctx->meta.p,
+              (size_t)rzk::kStatusWords, 0u);
+    RZ_TRY(enqueue_atlas_direct(ctx, s, rule, mode, fl, d_atlas, row_stride, (rzk::Status*)ctx->meta.p));
+    RZ_LAUNCH(ctx, "k_status_merge", rzk::k_status_merge, dim3(1), dim3(64),
+              (const rzk::Status*)ctx->meta.p, ctx->acc_run);
+    return check_launch(ctx, "atlas, direct");
+  }
   const rz_dpath* d = s->all;
   if (ctx->line_cap == 0) {
     ctx->line_cap = line_cap_for(std::max<size_t>((size_t)d->n_slots * 16, 1 << 16));
@@ -1709,9 +1770,8 @@ rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, dou
             dim3((uint32_t)std::min<size_t>(blocks_for(meta_u32), 4096)), dim3(rzk::kBlock), meta,
             meta_u32, 0u);
   RZ_LAUNCH(ctx, "k_atlas_setup", rzk::k_atlas_setup, dim3(blocks_for(n)), dim3(rzk::kBlock),
-            (const rzk::AtlasSlot*)s->atlas_slots, n, mode, pi);
+            (const rzk::AtlasSlot*)s->atlas_slots, n, mode, direct, pi);
   rzk::Xform x{};
-  const double fl = 16.0 * flatness * flatness;
   rzk::LineBufs lb;
   uint32_t* bin_fill = meta + meta_u32 - (rzk::kParts + 1 + rzk::kLineParts);
   int dq, dc;
@@ -1742,6 +1802,7 @@ rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, dou
   RZ_LAUNCH(ctx, "k_scene_bd", rzk::k_scene_bd, dim3(n), dim3(64), (const rzk::PathInfo*)pi, bd,
             redge, (const rzk::Status*)st);
   RZ_TRY(enqueue_bin_place(ctx, b, lb.fill));
+  if (direct) RZ_TRY(enqueue_atlas_direct(ctx, s, rule, mode, fl, d_atlas, row_stride, st));
   rzk::AtlasFineArgs a;
   RZ_TRY(ensure(ctx, ctx->atlas_tiles, (size_t)ct * sizeof(rzk::AtlasTile)));
   RZ_LAUNCH(ctx, "k_atlas_tiles", rzk::k_atlas_tiles, dim3(blocks_for(ct)), dim3(rzk::kBlock),
@@ -1893,6 +1954,41 @@ __global__ void k_set_colors(rzk::ScenePath* sp, const float* colors, uint32_t n
     sp[i].paint.color = rzp::c4(colors[4 * i], colors[4 * i + 1], colors[4 * i + 2], colors[4 * i + 3]);
 }
 
+// Whether a glyph's mask can be made by k_atlas_direct, and the largest
+// flatness bound and coordinate of its transformed curves. The accumulators
+// must fit (two workgroups a CU), the coordinates be finite, and the winding
+// stay in int32 at 2^-20: a flattened quad crosses a row at most twice, a
+// cubic three times, a line once, which bounds any pixel's winding.
+struct DirectBound {
+  double flatness = 0.0, coord = 0.0;
+};
+bool direct_glyph(const rz_path* p, const rzk::AtlasSlot& a, DirectBound* out) {
+  if (rzk::direct_lds((size_t)a.w, (size_t)a.h) > rzk::kDirectLds) return false;
+  uint64_t crossings = p->n_subpaths;  // closing lines
+  for (uint32_t k = 0; k < p->n_segments; ++k) {
+    const int np = p->kinds[k] + 2;
+    crossings += p->kinds[k] + 1u;
+    const double* q = p->points + 2 * (size_t)p->point_offsets[k];
+    rzg::Node<4> n;
+    for (int i = 0; i < np; ++i) {
+      n.p[i] = rzg::tr_apply(a.m, rzg::mkpt(q[2 * i], q[2 * i + 1]));
+      const double c = std::fmax(std::fabs(n.p[i].x), std::fabs(n.p[i].y));
+      if (!(std::fabs(n.p[i].x) < 1e9 && std::fabs(n.p[i].y) < 1e9)) return false;
+      out->coord = std::max(out->coord, c);
+    }
+    double f = 0.0;
+    if (p->kinds[k] == RZ_QUAD) {
+      rzg::Node<3> t;
+      for (int i = 0; i < 3; ++i) t.p[i] = n.p[i];
+      f = rzk::flatness_bound(t);
+    } else if (p->kinds[k] == RZ_CUBIC) {
+      f = rzk::flatness_bound(n);
+    }
+    out->flatness = std::max(out->flatness, f);
+  }
+  return crossings < 2000;
+}
+
 rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) {
   if (!ctx || !s) return RZ_E_ARG;
   if (s->n && !slots) return fail(ctx, RZ_E_ARG, "slots is NULL");
@@ -1911,7 +2007,7 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
     a.tile_base = (uint32_t)t;
     a.band_base = (uint32_t)b;
     a.redge_base = (uint32_t)r;
-    a.pad = 0;
+    a.direct = 0;
     const uint64_t tx = (q.width + 15) / 16, ty = (q.height + 15) / 16;
     if (q.width && q.height) {
       t += tx * ty;
@@ -1921,9 +2017,45 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
   }
   if (t > 0xffffffffull || r > 0xffffffffull) return fail(ctx, RZ_E_ARG, "atlas too large");
   SplitSum sum;
+  std::vector<uint32_t> slot_begin(s->n + 1), list;
+  s->n_direct = s->n_binned = 0;
+  s->direct_bound = s->direct_coord = 0.0;
   for (uint32_t i = 0; i < s->n; ++i) {
     const rz_path hp = s->host_path(i);
     split_sum(&hp, slots[i].tr.m, &sum);
+    slot_begin[i + 1] = slot_begin[i] + hp.n_segments + hp.n_subpaths;
+    rzk::AtlasSlot& a = v[i];
+    if (!a.w || !a.h) continue;
+    DirectBound db;
+    if (direct_glyph(&hp, a, &db)) {
+      a.direct = 1;
+      list.push_back(i);
+      s->direct_bound = std::max(s->direct_bound, db.flatness);
+      s->direct_coord = std::max(s->direct_coord, db.coord);
+    } else {
+      ++s->n_binned;
+    }
+  }
+  s->n_direct = (uint32_t)list.size();
+  // size classes, the largest first (and within a class the longest paths):
+  // each is launched with the LDS of its largest glyph
+  auto lds_of = [&](uint32_t i) { return rzk::direct_lds((size_t)v[i].w, (size_t)v[i].h); };
+  auto class_of = [&](uint32_t i) {
+    const size_t b = lds_of(i);
+    return b <= ((size_t)6 << 10) ? 0 : b <= ((size_t)12 << 10) ? 1 : b <= ((size_t)24 << 10) ? 2
+           : b <= ((size_t)40 << 10) ? 3 : 4;
+  };
+  std::stable_sort(list.begin(), list.end(), [&](uint32_t x, uint32_t y) {
+    const int cx = class_of(x), cy = class_of(y);
+    if (cx != cy) return cx > cy;
+    return slot_begin[x + 1] - slot_begin[x] > slot_begin[y + 1] - slot_begin[y];
+  });
+  s->direct.clear();
+  for (uint32_t k = 0; k < s->n_direct; ++k) {
+    if (k == 0 || class_of(list[k]) != class_of(list[k - 1])) s->direct.push_back({k, 0, 0});
+    auto& c = s->direct.back();
+    ++c.count;
+    c.lds = std::max(c.lds, lds_of(list[k]));
   }
   s->atlas_est = sum.est();
   std::vector<uint32_t> tile_glyph(t);
@@ -1940,11 +2072,14 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
   s->atlas_tile_glyph = nullptr;
   Pack pk;
   const size_t o_slots = pk.put(v), o_glyph = pk.put(tile_glyph);
+  const size_t o_list = pk.put(list), o_begin = pk.put(slot_begin);
   void* base = nullptr;
   RZ_TRY(dev_alloc(ctx, s->atlas_allocs, pk.h.size(), &base));
   RZ_TRY(pk.copy(ctx, base));
   s->atlas_slots = (rzk::AtlasSlot*)((char*)base + o_slots);
   s->atlas_tile_glyph = (uint32_t*)((char*)base + o_glyph);
+  s->direct_list = (const uint32_t*)((char*)base + o_list);
+  s->direct_slots = (const uint32_t*)((char*)base + o_begin);
   s->atlas_tiles = (uint32_t)t;
   s->atlas_bands = (uint32_t)b;
   s->atlas_rows = (uint32_t)r;
@@ -2844,6 +2979,10 @@ rz_status rz_ctx_create(rz_ctx** out, int device) {
   if (e == hipSuccess) e = hipMalloc((void**)&ctx->acc, 2 * sizeof(rzk::Status));
   if (e == hipSuccess) e = hipMemset(ctx->acc, 0, 2 * sizeof(rzk::Status));
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->xev, hipEventDisableTiming);
+  // k_atlas_direct's accumulators may take more than 64 KB of LDS
+  for (const void* k : {(const void*)rzk::k_atlas_direct<0>, (const void*)rzk::k_atlas_direct<1>})
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rzk::kDirectLds);
   if (e == hipSuccess) ctx->scratch_ptr = noalloc_scratch(device);
   if (e == hipSuccess) {
     hipDeviceProp_t prop;
@@ -3672,6 +3811,12 @@ rz_status rz_mask_atlas(rz_ctx* ctx, const rz_path* const* paths, const rz_atlas
 rz_status rz_scene_update_device(rz_ctx* ctx, rz_dscene* scene, const double* d_points,
                                  const float* d_colors) {
   if (!ctx || !scene) return RZ_E_ARG;
+  if (d_points && scene->n_points && !scene->points_updated) {
+    // the glyphs' bounds were made from the host's points: no k_atlas_direct
+    // from now on, nor a frame captured with it
+    scene->points_updated = true;
+    if (scene->n_direct) scene->serial = g_serial.fetch_add(1);
+  }
   if (d_points && scene->n_points)
     RZ_HIP(ctx, hipMemcpyAsync((void*)scene->all->view.pts, d_points,
                                (size_t)scene->n_points * 2 * sizeof(double),

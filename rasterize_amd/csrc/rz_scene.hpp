@@ -788,17 +788,19 @@ namespace rzk {
 struct AtlasSlot {
   double m[6];
   int x, y, w, h;
-  uint32_t tile_base, band_base, redge_base, pad;
+  uint32_t tile_base, band_base, redge_base;
+  uint32_t direct;  // 1: masked by k_atlas_direct where the call allows it
 };
 
+// direct: the glyphs marked so are masked by k_atlas_direct, not here.
 __global__ __launch_bounds__(kBlock) void k_atlas_setup(const AtlasSlot* slots, uint32_t n, int mode,
-                                                         PathInfo* pi) {
+                                                         bool direct, PathInfo* pi) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   const AtlasSlot& s = slots[i];
   PathInfo P;
   for (int k = 0; k < 6; ++k) P.m[k] = s.m[k];
-  P.live = s.w > 0 && s.h > 0;
+  P.live = s.w > 0 && s.h > 0 && !(direct && s.direct);
   P.rule = 0;
   P.ox = s.x;
   P.oy = s.y;

@@ -1,0 +1,126 @@
+"""Glyphs masked in one workgroup (k_atlas_direct) against the oracle: mask
+sizes around 16-pixel columns, one pixel, and the largest the accumulators
+hold, next to glyphs that go through the tile pipeline (too large, too many
+segments), with lines, quads and cubics, long edges, paths crossing every side
+of their view, both edge modes and fill rules, more slots than are staged at
+once, and a flatness that needs the deepest subdivision.
+
+A pixel sums the deposits of the lines in it, each rounded once to 2^-20, of
+coordinates rounded to 2^-20 (heights) and 2^-23 (columns): 2e-5 holds for the
+twenty-odd lines a pixel sees here."""
+import numpy as np
+import pytest
+import torch
+
+import _oracle as O
+import rasterize_amd as rz
+from rasterize_amd import FillRule, PathBuilder, Transform
+
+pytestmark = pytest.mark.gpu
+
+BAR = 2e-5
+
+
+def blob(rng, w, h, n, kinds="lqc", over=0.0):
+    """n segments round the middle of a w x h view, reaching `over` beyond it."""
+    c = np.array([0.5 * w, 0.5 * h])
+    r = (0.5 + over) * np.array([w, h])
+    th = np.sort(rng.uniform(0, 2 * np.pi, n))
+    at = lambda t, k: tuple(c + k * r * np.array([np.cos(t), np.sin(t)]))  # noqa: E731
+    pb = PathBuilder().move_to(at(th[0], rng.uniform(0.4, 1.0)))
+    for k in range(n):
+        t = th[(k + 1) % n]
+        end = at(t, rng.uniform(0.4, 1.0))
+        kind = kinds[int(rng.integers(len(kinds)))]
+        if kind == "l":
+            pb.line_to(end)
+        elif kind == "q":
+            pb.quad_to(at(t - 0.1, rng.uniform(0.2, 1.2)), end)
+        else:
+            pb.cubic_to(at(t - 0.4, rng.uniform(0.2, 1.3)), at(t + 0.3, rng.uniform(0.2, 1.3)), end)
+    return pb.close().build()
+
+
+def check(paths, sizes, rule, mode, trs=None, flatness=0.05):
+    trs = trs or [Transform.identity()] * len(paths)
+    slots, x = [], 3
+    for (w, h), tr in zip(sizes, trs):
+        slots.append(rz.atlas_slot(x, 2, w, h, tr))
+        x += w + 1
+    atlas = np.full((max(h for _, h in sizes) + 5, x + 4), -1.0, np.float32)
+    inside = np.zeros(atlas.shape, bool)
+    rz.mask_atlas(paths, slots, atlas, rule, flatness=flatness, edge_mode=mode)
+    worst = 0.0
+    for p, s, tr in zip(paths, slots, trs):
+        f = O.sd_mask if mode == rz._abi.RZ_EDGE_MASK else O.sd_mask_iter
+        ref = f(p, tr, s.width, s.height, rule, flatness)
+        got = atlas[s.y:s.y + s.height, s.x:s.x + s.width]
+        d = np.abs(got - ref).max()
+        worst = max(worst, d)
+        assert d <= BAR, (s.width, s.height, d)
+        inside[s.y:s.y + s.height, s.x:s.x + s.width] = True
+    print(f"{len(paths)} glyphs, rule {rule}, mode {mode}: max|d|={worst:.2e}", flush=True)
+    assert (atlas[~inside] == -1.0).all()
+
+
+@pytest.mark.parametrize("rule", [FillRule.NonZero, FillRule.EvenOdd])
+@pytest.mark.parametrize("mode", [rz._abi.RZ_EDGE_MASK, rz._abi.RZ_EDGE_ITER])
+def test_sizes_and_sides(rule, mode):
+    rng = np.random.default_rng(11)
+    sizes = [(1, 1), (2, 5), (15, 16), (16, 17), (17, 33), (31, 1), (64, 64), (65, 3), (128, 128),
+             (133, 131), (200, 190), (40, 300)]
+    paths = [blob(rng, w, h, int(n), over=o) for (w, h), n, o in
+             zip(sizes, [3, 4, 9, 20, 127, 5, 129, 12, 300, 60, 40, 7], [0, .3, 0, .2, .1, .5, 0, .4, .05, .3, .1, 0])]
+    check(paths, sizes, rule, mode)
+
+
+def test_transforms_long_edges_and_many_segments():
+    rng = np.random.default_rng(12)
+    sizes = [(96, 120), (50, 40), (60, 60), (100, 90)]
+    paths = [blob(rng, 96, 120, 4, "l", 2.0), blob(rng, 50, 40, 6, "c", 3.0),
+             blob(rng, 60, 60, 1100, "qc", 0.1),  # more crossings than int32 allows for: tile pipeline
+             blob(rng, 100, 90, 30)]
+    trs = [Transform.identity(), Transform.new_rotate(0.4), Transform.identity(),
+           Transform.new_translate(20.0, -15.0) * Transform.new_scale(1.7, 0.6)]
+    for rule in (FillRule.NonZero, FillRule.EvenOdd):
+        check(paths, sizes, rule, rz._abi.RZ_EDGE_MASK, trs)
+
+
+@pytest.mark.parametrize("flatness", [1e-4, 0.01, 2.0])
+def test_flatness(flatness):
+    rng = np.random.default_rng(13)
+    check([blob(rng, 60, 50, 12), blob(rng, 30, 30, 5, "qc", 0.5)], [(60, 50), (30, 30)], FillRule.NonZero,
+          rz._abi.RZ_EDGE_MASK, flatness=flatness)
+
+
+def test_updated_points_and_not_a_number():
+    """Points replaced on the device are masked as they are; a NaN among the
+    uploaded ones is reported as the reference reports it."""
+    rng = np.random.default_rng(14)
+    a = blob(rng, 60, 50, 12, "q")
+    moved = a.points.copy().reshape(-1, 3, 2)  # the quads' control points; their ends stay joined
+    moved[:, 1] += rng.uniform(-25.0, 25.0, moved[:, 1].shape)
+    b = rz.Path(a.kinds, a.point_offsets, moved, a.subpaths, a.closed)
+    glyphs = rz.DeviceGlyphs([a], [rz.atlas_slot(0, 0, 60, 50)])
+    out = torch.zeros((50, 60), device="cuda")
+
+    def run():
+        for _ in range(4):
+            glyphs.mask_device(out.data_ptr(), 60)
+            try:
+                glyphs.ctx.sync()
+                return out.cpu().numpy()
+            except rz.RzError as e:
+                assert e.status == rz._abi.RZ_E_CAPACITY
+    torch.cuda.synchronize()
+    assert np.abs(run() - O.sd_mask(a, Transform.identity(), 60, 50, 0)).max() <= BAR
+    pts = torch.tensor(b.points, device="cuda")
+    torch.cuda.synchronize()
+    glyphs.ctx.check(rz._abi.lib().rz_scene_update_device(glyphs.ctx.h, glyphs.h, pts.data_ptr(), None))
+    assert np.abs(run() - O.sd_mask(b, Transform.identity(), 60, 50, 0)).max() <= BAR
+    bad = blob(rng, 60, 50, 12, "q")
+    bad.points[7] = np.nan
+    with pytest.raises(rz.RzError) as e:
+        rz.mask_atlas([a, bad], [rz.atlas_slot(0, 0, 60, 50), rz.atlas_slot(60, 0, 60, 50)],
+                      np.zeros((50, 120), np.float32))
+    assert e.value.status == rz._abi.RZ_E_NAN
