@@ -1211,6 +1211,7 @@ struct rz_dscene {
   const uint32_t* direct_list = nullptr;
   const uint32_t* direct_slots = nullptr;  // [n + 1] first flatten slot of each glyph
   double direct_bound = 0.0, direct_coord = 0.0;  // largest flatness bound and coordinate
+  bool direct_cubics = false;            // some of them have cubics
   bool points_updated = false;           // the device's points are not the host's any more
   // host copies of the paths, one after the other: for Path::bbox(tr) and the
   // resident paths of the plain form, and the atlas's line estimate
@@ -1682,7 +1683,7 @@ rz_status enqueue_scene_plain(rz_ctx* ctx, const rz_dscene* s, const rz_transfor
 
 // The glyphs of k_atlas_direct. Few glyphs go in one launch with the LDS of
 // the largest (two workgroups a CU hold them all at once); more in a launch per
-// size class, so that small glyphs are not held to the largest one's occupancy.
+// size class (kDirectSmall).
 rz_status enqueue_atlas_direct(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, double fl,
                                float* d_atlas, size_t row_stride, rzk::Status* st) {
   rzk::DirectArgs a;
@@ -1694,21 +1695,28 @@ rz_status enqueue_atlas_direct(rz_ctx* ctx, const rz_dscene* s, int rule, int mo
   a.out = d_atlas;
   a.row_stride = row_stride;
   a.st = st;
-  auto launch = [&](uint32_t first, uint32_t count, size_t lds) {
+  auto launch = [&](uint32_t first, uint32_t count, size_t lds, uint32_t threads) {
     a.list = s->direct_list + first;
-    if (rule == RZ_NONZERO)
-      RZ_LAUNCH_LDS(ctx, "k_atlas_direct<0>", rzk::k_atlas_direct<0>, dim3(count),
-                    dim3(rzk::kDirectBlock), lds, a);
-    else
-      RZ_LAUNCH_LDS(ctx, "k_atlas_direct<1>", rzk::k_atlas_direct<1>, dim3(count),
-                    dim3(rzk::kDirectBlock), lds, a);
+    const dim3 grid(count), block(threads);
+    if (rule == RZ_NONZERO) {
+      if (s->direct_cubics)
+        RZ_LAUNCH_LDS(ctx, "k_atlas_direct<0>", (rzk::k_atlas_direct<0, true>), grid, block, lds, a);
+      else
+        RZ_LAUNCH_LDS(ctx, "k_atlas_direct<0>", (rzk::k_atlas_direct<0, false>), grid, block, lds, a);
+    } else {
+      if (s->direct_cubics)
+        RZ_LAUNCH_LDS(ctx, "k_atlas_direct<1>", (rzk::k_atlas_direct<1, true>), grid, block, lds, a);
+      else
+        RZ_LAUNCH_LDS(ctx, "k_atlas_direct<1>", (rzk::k_atlas_direct<1, false>), grid, block, lds, a);
+    }
   };
   if (s->n_direct <= 2 * (uint32_t)ctx->n_cus) {
     size_t lds = 0;
     for (const auto& c : s->direct) lds = std::max(lds, c.lds);
-    launch(0, s->n_direct, lds);
+    launch(0, s->n_direct, lds, rzk::kDirectBlock);
   } else {
-    for (const auto& c : s->direct) launch(c.first, c.count, c.lds);
+    for (const auto& c : s->direct)
+      launch(c.first, c.count, c.lds, c.lds <= rzk::kDirectSmall ? 128 : 256);
   }
   return check_launch(ctx, "k_atlas_direct");
 }
@@ -1961,6 +1969,7 @@ __global__ void k_set_colors(rzk::ScenePath* sp, const float* colors, uint32_t n
 // cubic three times, a line once, which bounds any pixel's winding.
 struct DirectBound {
   double flatness = 0.0, coord = 0.0;
+  bool cubics = false;
 };
 bool direct_glyph(const rz_path* p, const rzk::AtlasSlot& a, DirectBound* out) {
   if (rzk::direct_lds((size_t)a.w, (size_t)a.h) > rzk::kDirectLds) return false;
@@ -1983,6 +1992,7 @@ bool direct_glyph(const rz_path* p, const rzk::AtlasSlot& a, DirectBound* out) {
       f = rzk::flatness_bound(t);
     } else if (p->kinds[k] == RZ_CUBIC) {
       f = rzk::flatness_bound(n);
+      out->cubics = true;
     }
     out->flatness = std::max(out->flatness, f);
   }
@@ -2020,6 +2030,7 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
   std::vector<uint32_t> slot_begin(s->n + 1), list;
   s->n_direct = s->n_binned = 0;
   s->direct_bound = s->direct_coord = 0.0;
+  s->direct_cubics = false;
   for (uint32_t i = 0; i < s->n; ++i) {
     const rz_path hp = s->host_path(i);
     split_sum(&hp, slots[i].tr.m, &sum);
@@ -2032,6 +2043,7 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
       list.push_back(i);
       s->direct_bound = std::max(s->direct_bound, db.flatness);
       s->direct_coord = std::max(s->direct_coord, db.coord);
+      s->direct_cubics = s->direct_cubics || db.cubics;
     } else {
       ++s->n_binned;
     }
@@ -2040,11 +2052,7 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
   // size classes, the largest first (and within a class the longest paths):
   // each is launched with the LDS of its largest glyph
   auto lds_of = [&](uint32_t i) { return rzk::direct_lds((size_t)v[i].w, (size_t)v[i].h); };
-  auto class_of = [&](uint32_t i) {
-    const size_t b = lds_of(i);
-    return b <= ((size_t)6 << 10) ? 0 : b <= ((size_t)12 << 10) ? 1 : b <= ((size_t)24 << 10) ? 2
-           : b <= ((size_t)40 << 10) ? 3 : 4;
-  };
+  auto class_of = [&](uint32_t i) { return lds_of(i) <= rzk::kDirectSmall ? 0 : 1; };
   std::stable_sort(list.begin(), list.end(), [&](uint32_t x, uint32_t y) {
     const int cx = class_of(x), cy = class_of(y);
     if (cx != cy) return cx > cy;
@@ -2980,7 +2988,8 @@ rz_status rz_ctx_create(rz_ctx** out, int device) {
   if (e == hipSuccess) e = hipMemset(ctx->acc, 0, 2 * sizeof(rzk::Status));
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->xev, hipEventDisableTiming);
   // k_atlas_direct's accumulators may take more than 64 KB of LDS
-  for (const void* k : {(const void*)rzk::k_atlas_direct<0>, (const void*)rzk::k_atlas_direct<1>})
+  for (const void* k : {(const void*)rzk::k_atlas_direct<0, false>, (const void*)rzk::k_atlas_direct<0, true>,
+                        (const void*)rzk::k_atlas_direct<1, false>, (const void*)rzk::k_atlas_direct<1, true>})
     if (e == hipSuccess)
       e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rzk::kDirectLds);
   if (e == hipSuccess) ctx->scratch_ptr = noalloc_scratch(device);

@@ -7,15 +7,25 @@
 
 namespace rzk {
 
-constexpr int kDirectBlock = 256;
+constexpr int kDirectBlock = 512;  // threads at most (and at least kDirectSlots)
 constexpr int kDirectSlots = 128;  // slots staged at once
 constexpr int kDirectDepth = 10;   // subdivision depth at most (checked on the host)
 // LDS of the accumulators at most: two workgroups per CU
 constexpr size_t kDirectLds = 70 << 10;
 
-// Accumulators: H rows of W | 1 ints (odd: neighbouring rows in different
-// banks), 2^-20 fixed point.
-inline size_t direct_lds(size_t W, size_t H) { return (W | 1) * H * sizeof(int); }
+// Accumulators: H rows of direct_stride(W) ints, 2^-20 fixed point; four
+// columns are a 16-byte read, and the odd number of them keeps neighbouring
+// rows in different banks.
+RZ_HD int direct_stride(int W) { return (((W + 3) >> 2) | 1) << 2; }
+inline size_t direct_lds(size_t W, size_t H) { return (size_t)direct_stride((int)W) * H * sizeof(int); }
+
+// Glyphs up to this size (24 KB: 76x76) are launched apart from larger ones,
+// with two waves a workgroup instead of four. 16,384 glyphs of 16 to 128 px:
+// these two classes 707 us, one class 792 (four waves) or 1079 (two), five
+// classes 766 to 893, eight waves 1228. A set that the chip holds at once is
+// one launch of eight waves a glyph, the shortest way through one: 400 glyphs
+// 42 us, 46 with four waves, 77 with two.
+constexpr size_t kDirectSmall = 24 << 10;
 
 // A bound on the flatness of a curve's nodes: at depth k of its subdivision
 // none is above bound / 16^k. A quad's second difference
@@ -86,26 +96,22 @@ __device__ inline void to_child(rzg::Node<4>& n, bool r) {
   n.p[2] = sel(r, outer, inner);
 }
 
-// The leaf of the root's subdivision along the depth bits `bits`: the chord,
-// if this thread owns it (a leaf above `depth` belongs to the bits that end in
-// zeros). The same nodes, tests and leaves as PathFlattenIter's.
+// One lane's part of a curve's subdivision (PathFlattenIter's nodes, tests and
+// leaves): the node reached from the root along `bits` (most significant
+// first) in `levels` levels, and its leaves below. A curve's leaves lie at
+// depth levels + 2 at most (leaf_depth), so they are the node itself, its
+// children or its grandchildren.
+enum { SUB_NONE = 0, SUB_LEAF = 1, SUB_SPLIT = 2 };
 template <int NP>
-__device__ inline bool leaf_line(const double2* root, uint32_t bits, int depth, double fl, Pt* a,
-                                 Pt* b, bool* deep) {
-  rzg::Node<NP> n;
+__device__ inline int sub_node(const double2* root, uint32_t bits, int levels, double fl,
+                               rzg::Node<NP>* n) {
 #pragma unroll
-  for (int i = 0; i < NP; ++i) n.p[i] = rzg::mkpt(root[i].x, root[i].y);
-  for (int left = depth;; --left) {
-    if (rzg::flatness(n) < fl) {
-      *a = n.p[0];
-      *b = n.p[NP - 1];
-      return (bits & ((1u << left) - 1u)) == 0;
-    }
-    if (left == 0) {
-      *deep = true;
-      return false;
-    }
-    to_child(n, (bits >> (left - 1)) & 1u);
+  for (int i = 0; i < NP; ++i) n->p[i] = rzg::mkpt(root[i].x, root[i].y);
+  for (int left = levels;; --left) {
+    // a leaf above the node belongs to the bits that end in zeros
+    if (rzg::flatness(*n) < fl) return (bits & ((1u << left) - 1u)) == 0 ? SUB_LEAF : SUB_NONE;
+    if (left == 0) return SUB_SPLIT;
+    to_child(*n, (bits >> (left - 1)) & 1u);
   }
 }
 
@@ -118,11 +124,52 @@ struct DirectMask {
   }
 };
 
-// A piece prepared for its row steps: lower end first.
+// Heights are rounded to 2^-20 of a pixel once per vertex (relative to any
+// pixel row: the same everywhere), and a row's total deposit is the difference
+// of two such heights, so that what the lines of a closed chain deposit in a
+// row cancels exactly to the right of them.
+__device__ inline int fix_height(double y) { return __double2int_rn(y * (double)(1 << rzg::kFixShift)); }
+
+// The deposits of a piece with total D (2^-20) in pixel row r, from column c +
+// u to c + v (0 <= u < 1): each column its share of the exact area, the last
+// one what the others leave of D. Without a branch up to two columns, which
+// nearly all lines of a flattened curve stay in; the reciprocal's error (one
+// unit in the last place) is below the rounding to 2^-20.
+__device__ inline void direct_cols(const DirectMask& M, int r, int c, float u, float v, int D) {
+  const float d = (float)D;
+  if (v > 2.0f) {
+    // the mean coverage of each column by the piece, differenced
+    const float s = 1.0f / (v - u);
+    const int n = (int)ceilf(v);  // columns c .. c + n - 1 are crossed
+    int sum = __float2int_rn(d * (0.5f * s * (1.0f - u) * (1.0f - u)));
+    M.add(r, c, sum);
+    for (int k = 1; k < n; ++k) {
+      const float e = fminf((float)(k + 1), v);
+      const float in = s * (e - (float)k);  // share of the piece inside column k
+      const float cov = s * ((float)k - u) + in * (1.0f - 0.5f * (e - (float)k));
+      const int A = __float2int_rn(d * cov) - sum;
+      M.add(r, c + k, A);
+      sum += A;
+    }
+    M.add(r, c + n, D - sum);
+    return;
+  }
+  const bool one = v <= 1.0f;
+  const float s = __builtin_amdgcn_rcpf(v - u), p = 1.0f - u, e = v - 1.0f;
+  const float cov0 = one ? 1.0f - 0.5f * (u + v) : 0.5f * p * p * s;
+  const int A0 = __float2int_rn(d * cov0);
+  const int A1 = one ? D - A0 : __float2int_rn(d * ((p + e * (1.0f - 0.5f * e)) * s)) - A0;
+  const int A2 = D - A0 - A1;
+  M.add(r, c, A0);
+  M.add(r, c + 1, A1);
+  if (A2) M.add(r, c + 2, A2);
+}
+
+// A piece of a line with 0 <= x <= W, lower end first.
 struct DirectPiece {
   double x0, y0, x1, y1;
-  int dir;  // +-1, 0: nothing to deposit
-  int r0, r1;
+  int dir;     // +-1
+  int r0, r1;  // pixel rows [r0, r1), none: nothing to deposit
 };
 
 __device__ inline DirectPiece direct_piece(Pt a, Pt b, int H) {
@@ -135,75 +182,70 @@ __device__ inline DirectPiece direct_piece(Pt a, Pt b, int H) {
   q.dir = up ? -1 : 1;
   const double lo = fmax(q.y0, 0.0), hi = fmin(q.y1, (double)H);
   q.r0 = q.r1 = 0;
-  if (!(lo < hi)) {
-    q.dir = 0;
-    return q;
+  if (lo < hi) {
+    q.r0 = (int)floor(lo);
+    q.r1 = (int)ceil(hi);
   }
-  q.r0 = (int)floor(lo);
-  q.r1 = (int)ceil(hi);
   return q;
 }
 
-// The deposits of the piece in pixel row r (0 <= x <= W). Positions are f64,
-// the fractions inside the row's pixels f32. The row's total is the difference
-// of its ends' heights in fixed point, so that what neighbouring lines of a
-// closed chain deposit cancels exactly to the right of them; the last column
-// takes what the others leave of it.
+// A short piece, by its lane: at most four rows and 16 columns, so that f32
+// positions relative to its first row and column are exact to 2^-20.
+__device__ inline void direct_short(const DirectMask& M, const DirectPiece& q) {
+  const double xl = floor(fmin(q.x0, q.x1)), yr = (double)q.r0;
+  const float x0 = (float)(q.x0 - xl), x1 = (float)(q.x1 - xl);
+  const int Y0 = fix_height(q.y0 - yr), Y1 = fix_height(q.y1 - yr);
+  const int c0 = (int)xl;
+  constexpr int one = 1 << rzg::kFixShift;
+  // per 2^-20 of a row; over at most four rows the reciprocal's error moves x
+  // by less than 2^-20
+  const float slope = Y1 > Y0 ? (x1 - x0) * __builtin_amdgcn_rcpf((float)(Y1 - Y0)) : 0.0f;
+  for (int r = q.r0; r < q.r1; ++r) {
+    const int ry = (r - q.r0) << rzg::kFixShift;
+    const int top = max(Y0, ry), bot = min(Y1, ry + one);
+    const float xt = x0 + slope * (float)(top - Y0);
+    const float xb = bot == Y1 ? x1 : x0 + slope * (float)(bot - Y0);
+    const float lo = fmaxf(fminf(xt, xb), 0.0f);
+    const float fl = floorf(lo);
+    direct_cols(M, r, c0 + (int)fl, lo - fl, fmaxf(xt, xb) - fl, q.dir * (bot - top));
+  }
+}
+
+// One row of a longer piece, positions in f64.
 __device__ inline void direct_row(const DirectMask& M, const DirectPiece& q, double dxdy, int r) {
   const double rt = (double)r, rb = rt + 1.0;
   const bool in0 = q.y0 >= rt, in1 = q.y1 <= rb;  // the ends lie in this row
   const double xt = in0 ? q.x0 : q.x0 + dxdy * (rt - q.y0);
   const double xb = in1 ? q.x1 : q.x0 + dxdy * (rb - q.y0);
-  const int f0 = in0 ? __float2int_rn((float)(q.y0 - rt) * kFix) : 0;
-  const int f1 = in1 ? __float2int_rn((float)(q.y1 - rt) * kFix) : 1 << rzg::kFixShift;
-  const int D = q.dir * (f1 - f0);
+  const int f0 = in0 ? fix_height(q.y0 - rt) : 0, f1 = in1 ? fix_height(q.y1 - rt) : 1 << rzg::kFixShift;
   const double xl = floor(fmax(fmin(xt, xb), 0.0));
-  const int c = (int)xl;
-  const float u = (float)(fmin(xt, xb) - xl), v = (float)(fmax(xt, xb) - xl);
-  const float d = (float)D;
-  if (v <= 1.0f) {
-    const int A = __float2int_rn(d * (1.0f - 0.5f * (u + v)));
-    M.add(r, c, A);
-    M.add(r, c + 1, D - A);
-    return;
-  }
-  // several columns: the area left of each column's right edge, differenced
-  const float s = 1.0f / (v - u);
-  const int n = (int)ceilf(v);  // columns c .. c + n - 1 are crossed
-  float prev = 0.5f * s * (1.0f - u) * (1.0f - u);
-  int sum = __float2int_rn(d * prev);
-  M.add(r, c, sum);
-  for (int k = 1; k < n; ++k) {
-    // mean coverage of column k by the piece: exact trapezoid, 1 past its end
-    const float e = fminf((float)(k + 1), v);
-    const float in = s * (e - (float)k);                       // share of the piece inside
-    const float cov = s * ((float)k - u) + in * (1.0f - 0.5f * (e - (float)k));
-    const int A = __float2int_rn(d * cov) - sum;
-    M.add(r, c + k, A);
-    sum += A;
-  }
-  M.add(r, c + n, D - sum);
+  direct_cols(M, r, (int)xl, (float)(fmax(fmin(xt, xb), 0.0) - xl), (float)(fmax(xt, xb) - xl), q.dir * (f1 - f0));
 }
 
 // A line per lane (have) into the accumulators: right clip and left split
-// (rzg::effective_line), then each piece's rows: up to four by the lane
-// itself, more by the whole wave. Every lane takes part.
+// (rzg::effective_line) where a lane's line needs them, short pieces by their
+// lanes, longer ones row by row by the whole wave. Every lane takes part.
 __device__ inline void direct_line(const DirectMask& M, const rzg::BinGrid& g, bool have, Pt a, Pt b,
                                    int lane) {
-  rzg::EffLine e;
-  e.n = 0;
-  if (have) e = rzg::effective_line(a, b, g);
-  for (int pc = 0; __ballot(pc < e.n); ++pc) {
+  int left = have ? 1 : 0;  // pieces left: (a, b), then (b, c)
+  Pt c = b;
+  if (have && !(fmin(a.x, b.x) >= 0.0 && fmax(a.x, b.x) <= g.wc)) {
+    const rzg::EffLine e = rzg::effective_line(a, b, g);
+    left = e.n;
+    a = e.p[0];
+    b = e.p[1];
+    c = e.p[2];
+  }
+  for (; __ballot(left > 0); --left, a = b, b = c) {
     DirectPiece q;
-    q.dir = 0;
+    q.x0 = q.y0 = q.x1 = q.y1 = 0.0;
+    q.dir = 1;
     q.r0 = q.r1 = 0;
-    if (pc < e.n) q = direct_piece(pc ? e.p[1] : e.p[0], pc ? e.p[2] : e.p[1], M.H);
+    if (left > 0) q = direct_piece(a, b, M.H);
     const int rows = q.r1 - q.r0;
-    double dxdy = 0.0;
-    if (q.dir && (rows > 1 || q.y0 < 0.0 || q.y1 > (double)M.H)) dxdy = (q.x1 - q.x0) / (q.y1 - q.y0);
-    if (q.dir && rows <= 4)
-      for (int r = q.r0; r < q.r1; ++r) direct_row(M, q, dxdy, r);
-    uint64_t m = __ballot(q.dir && rows > 4);
+    const bool small = rows <= 4 && fabs(q.x1 - q.x0) <= 16.0 && q.y1 - q.y0 <= 16.0;
+    if (rows > 0 && small) direct_short(M, q);
+    uint64_t m = __ballot(rows > 0 && !small);
     while (m) {
       const int src = __ffsll((unsigned long long)m) - 1;
       m &= m - 1;
@@ -219,29 +261,33 @@ __device__ inline void direct_line(const DirectMask& M, const rzg::BinGrid& g, b
       w.dir = __builtin_amdgcn_readlane(q.dir, src);
       w.r0 = __builtin_amdgcn_readlane(q.r0, src);
       w.r1 = __builtin_amdgcn_readlane(q.r1, src);
-      const double s = of(dxdy);
-      for (int r = w.r0 + lane; r < w.r1; r += 64) direct_row(M, w, s, r);
+      const double dxdy = (w.x1 - w.x0) / (w.y1 - w.y0);
+      for (int r = w.r0 + lane; r < w.r1; r += 64) direct_row(M, w, dxdy, r);
     }
   }
 }
 
 // One glyph per workgroup. Its slots are staged kDirectSlots at a time with
-// their control points under the glyph's transform; the leaves of all staged
-// curves at their deepest level are dealt out to the lanes, each of which
-// walks from the root to its leaf (three or four levels for a glyph's curves:
-// less work than a depth-first walk whose lanes wait for the longest subtree)
-// and deposits the line. Then a wave sums four rows at a time, 16 pixels each,
-// and writes the mask.
-// Bound by VALU issue. DIRECT
-template <int RULE>
+// their control points under the glyph's transform. The subdivision nodes two
+// levels above the deepest leaves (fewer where that leaves lanes idle) are
+// dealt out to the lanes; a lane walks to its node (one or two levels for a
+// glyph's curves) and deposits the up to four lines below it: no depth-first
+// walk whose lanes wait for the longest subtree. Then a wave sums four rows at
+// a time, 64 pixels each, and writes the mask.
+// Bound by latency and VALU issue (40% of the SIMD cycles). Against the tile
+// pipeline: 400 glyphs 114 -> 43 us, 16,384 glyphs 1178 -> 707 us.
+// CUBIC: some path has cubics (a TrueType font's have none, and the kernel
+// without them fits four waves per SIMD).
+template <int RULE, bool CUBIC>
 __global__ __launch_bounds__(kDirectBlock) void k_atlas_direct(DirectArgs a) {
-  extern __shared__ int acc[];
+  extern __shared__ int4 acc4[];
+  int* acc = (int*)acc4;
   __shared__ double2 pts[kDirectSlots][4];
   __shared__ uint32_t pre[kDirectSlots + 1];
   __shared__ uint32_t kd[kDirectSlots];  // kind | depth << 8
-  __shared__ uint32_t half_total;
+  __shared__ uint32_t half_total, nodes2[2];
   __shared__ int marks_all[kDirectBlock / 64][64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = (int)blockDim.x;
   int* marks = marks_all[wave];
   const uint32_t glyph = load_const(a.list + blockIdx.x);
   const AtlasSlot S = load_const(a.slots + glyph);
@@ -250,14 +296,14 @@ __global__ __launch_bounds__(kDirectBlock) void k_atlas_direct(DirectArgs a) {
   g.W = S.w;
   g.H = S.h;
   g.wc = a.mode == rzg::EDGE_MASK ? (double)S.w - 1.0 : (double)S.w;
-  const DirectMask M{acc, S.w | 1, S.w, S.h};
-  for (int i = tid; i < M.H * M.stride; i += kDirectBlock) acc[i] = 0;
+  const DirectMask M{acc, direct_stride(S.w), S.w, S.h};
+  for (int i = tid; i < M.H * (M.stride / 4); i += nt) ((int4*)acc)[i] = make_int4(0, 0, 0, 0);
   const uint32_t s_end = load_const(a.slot_begin + glyph + 1);
   uint32_t lines = 0;
   bool deep = false;
   for (uint32_t s0 = load_const(a.slot_begin + glyph); s0 < s_end; s0 += kDirectSlots) {
     __syncthreads();  // the previous slots have been read
-    uint32_t n = 0;
+    int my_depth = -1;
     if (tid < kDirectSlots) {
       const uint32_t slot = s0 + (uint32_t)tid;
       if (slot < s_end) {
@@ -283,7 +329,7 @@ __global__ __launch_bounds__(kDirectBlock) void k_atlas_direct(DirectArgs a) {
             t.p[1] = q.p[1];
             t.p[2] = q.p[2];
             depth = leaf_depth(flatness_bound(t), a.fl);
-          } else if (kind == rzg::KIND_CUBIC) {
+          } else if (CUBIC && kind == rzg::KIND_CUBIC) {
             depth = leaf_depth(flatness_bound(q), a.fl);
           }
           if (depth > kDirectDepth) {
@@ -292,8 +338,18 @@ __global__ __launch_bounds__(kDirectBlock) void k_atlas_direct(DirectArgs a) {
           }
         }
         kd[tid] = (uint32_t)kind | (uint32_t)depth << 8;
-        n = 1u << depth;
+        my_depth = depth;
       }
+      uint32_t total;
+      (void)wave_excl_scan(my_depth < 0 ? 0u : 1u << max(my_depth - 2, 0), lane, &total);
+      if (lane == 0) nodes2[wave] = total;
+    }
+    __syncthreads();
+    // levels a lane takes below its node
+    const uint32_t n2 = nodes2[0] + nodes2[1];
+    const int below = n2 * 4u <= (uint32_t)nt ? 0 : n2 * 2u <= (uint32_t)nt ? 1 : 2;
+    if (tid < kDirectSlots) {
+      const uint32_t n = my_depth < 0 ? 0u : 1u << max(my_depth - below, 0);
       uint32_t total;
       const uint32_t ex = wave_excl_scan(n, lane, &total);
       pre[tid] = ex;
@@ -307,8 +363,8 @@ __global__ __launch_bounds__(kDirectBlock) void k_atlas_direct(DirectArgs a) {
     const uint32_t total = pre[kDirectSlots];
     const uint32_t p0 = pre[lane], p1 = pre[64 + lane];
     const bool v0 = pre[lane + 1] > p0, v1 = pre[65 + lane] > p1;
-    for (uint32_t j0 = (uint32_t)wave * 64u; j0 < total; j0 += kDirectBlock) {
-      // owner of leaf j0 + lane: the last slot that starts at or before it
+    for (uint32_t j0 = (uint32_t)wave * 64u; j0 < total; j0 += (uint32_t)nt) {
+      // owner of node j0 + lane: the last slot that starts at or before it
       marks[lane] = -1;
       wave_lds_sync();
       if (v0 && p0 >= j0 && p0 - j0 < 64u) marks[p0 - j0] = lane;
@@ -318,49 +374,107 @@ __global__ __launch_bounds__(kDirectBlock) void k_atlas_direct(DirectArgs a) {
       wave_lds_sync();
       const int o = max(dpp_max_scan(marks[lane]), first);
       const uint32_t j = j0 + (uint32_t)lane;
-      Pt u = rzg::mkpt(0.0, 0.0), v = u;
-      bool have = false;
-      if (j < total) {
-        const uint32_t bits = j - pre[o], q = kd[o];
-        const int kind = (int)(q & 255u), depth = (int)(q >> 8);
-        if (kind == rzg::KIND_QUAD) {
-          have = leaf_line<3>(pts[o], bits, depth, a.fl, &u, &v, &deep);
-        } else if (kind == rzg::KIND_CUBIC) {
-          have = leaf_line<4>(pts[o], bits, depth, a.fl, &u, &v, &deep);
-        } else {
-          u = rzg::mkpt(pts[o][0].x, pts[o][0].y);
-          v = rzg::mkpt(pts[o][1].x, pts[o][1].y);
-          have = true;
+      int sub = SUB_NONE;
+      const uint32_t q = kd[o];
+      const int kind = j < total ? (int)(q & 255u) : -1;
+      rzg::Node<4> n;  // a line's or quad's points in the first two or three
+#pragma unroll
+      for (int i = 0; i < 4; ++i) n.p[i] = rzg::mkpt(0.0, 0.0);
+      const int levels = max((int)(q >> 8) - below, 0);
+      if (kind == rzg::KIND_QUAD) {
+        rzg::Node<3> t;
+        sub = sub_node(pts[o], j - pre[o], levels, a.fl, &t);
+        n.p[0] = t.p[0];
+        n.p[1] = t.p[1];
+        n.p[2] = t.p[2];
+      } else if (CUBIC && kind == rzg::KIND_CUBIC) {
+        sub = sub_node(pts[o], j - pre[o], levels, a.fl, &n);
+      } else if (kind == rzg::KIND_LINE) {
+        n.p[0] = rzg::mkpt(pts[o][0].x, pts[o][0].y);
+        n.p[1] = rzg::mkpt(pts[o][1].x, pts[o][1].y);
+        sub = SUB_LEAF;
+      }
+      // the node's chord, or its children's, or its grandchildren's
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) {
+        if (h && !__ballot(sub == SUB_SPLIT)) break;
+        rzg::Node<4> c = n;
+        bool leaf = true;  // c's chord is one of the lines
+        if (sub == SUB_SPLIT) {
+          if (!CUBIC || kind == rzg::KIND_QUAD) {
+            rzg::Node<3> t;
+            t.p[0] = n.p[0];
+            t.p[1] = n.p[1];
+            t.p[2] = n.p[2];
+            to_child(t, h != 0);
+            leaf = rzg::flatness(t) < a.fl;
+            c.p[0] = t.p[0];
+            c.p[1] = t.p[1];
+            c.p[2] = t.p[2];
+          } else {
+            to_child(c, h != 0);
+            leaf = rzg::flatness(c) < a.fl;
+          }
+        }
+#pragma unroll 1
+        for (int k = 0; k < 2; ++k) {
+          bool have = sub == SUB_SPLIT || (sub == SUB_LEAF && h == 0);
+          if (leaf && k) have = false;
+          if (!__ballot(have)) break;
+          Pt u = c.p[0], v = CUBIC && kind == rzg::KIND_CUBIC ? c.p[3] : kind == rzg::KIND_QUAD ? c.p[2] : c.p[1];
+          if (have && !leaf) {
+            if (!CUBIC || kind == rzg::KIND_QUAD) {
+              rzg::Node<3> t;
+              t.p[0] = c.p[0];
+              t.p[1] = c.p[1];
+              t.p[2] = c.p[2];
+              to_child(t, k != 0);
+              deep = deep || !(rzg::flatness(t) < a.fl);
+              u = t.p[0];
+              v = t.p[2];
+            } else {
+              rzg::Node<4> t = c;
+              to_child(t, k != 0);
+              deep = deep || !(rzg::flatness(t) < a.fl);
+              u = t.p[0];
+              v = t.p[3];
+            }
+          }
+          lines += (uint32_t)__popcll(__ballot(have));
+          direct_line(M, g, have, u, v, lane);
         }
       }
-      lines += (uint32_t)__popcll(__ballot(have));
-      direct_line(M, g, have, u, v, lane);
     }
   }
   if (deep) set_err(a.st, rzg::ST_DEPTH);
   if (lane == 0 && lines) atomicAdd(&a.st->n_lines, lines);
   __syncthreads();
-  // row sums: 16 lanes a row, 16 columns at a time, the sum so far carried
-  // from lane 15 to lane 0 (row_ror:1)
-  const int col = lane & 15;
-  const int first_lane = col == 0 ? -1 : 0;
-  for (int r0 = wave * 4; r0 < M.H; r0 += 4 * (kDirectBlock / 64)) {
+  // row sums: 16 lanes a row, four columns a lane; the sum so far carried from
+  // lane 15 to lane 0 (row_ror:1)
+  const int first_lane = (lane & 15) == 0 ? -1 : 0;
+  for (int r0 = wave * 4; r0 < M.H; r0 += nt >> 4) {
     const int r = r0 + (lane >> 4);
     const bool in = r < M.H;
     const int* row = acc + r * M.stride;
     float* out = a.out + (size_t)(S.y + r) * a.row_stride + S.x;
     int run = 0;
-    for (int c0 = 0; c0 < M.W; c0 += 16) {
-      const int c = c0 + col;
-      const bool px = in && c < M.W;
-      int w = px ? row[c] : 0;
-      w += __builtin_amdgcn_update_dpp(0, run, 0x121, 0xf, 0xf, false) & first_lane;
-      w += __builtin_amdgcn_update_dpp(0, w, 0x111, 0xf, 0xf, false);
-      w += __builtin_amdgcn_update_dpp(0, w, 0x112, 0xf, 0xf, false);
-      w += __builtin_amdgcn_update_dpp(0, w, 0x114, 0xf, 0xf, false);
-      w += __builtin_amdgcn_update_dpp(0, w, 0x118, 0xf, 0xf, false);
-      run = w;
-      if (px) out[c] = alpha_fix<RULE>(w);
+    for (int c0 = 0; c0 < M.W; c0 += 64) {
+      const int c = c0 + ((lane & 15) << 2);
+      int4 w = make_int4(0, 0, 0, 0);
+      if (in && c < M.W) w = *(const int4*)(row + c);
+      w.y += w.x;
+      w.z += w.y;
+      w.w += w.z;
+      int t = w.w + (__builtin_amdgcn_update_dpp(0, run, 0x121, 0xf, 0xf, false) & first_lane);
+      t += __builtin_amdgcn_update_dpp(0, t, 0x111, 0xf, 0xf, false);
+      t += __builtin_amdgcn_update_dpp(0, t, 0x112, 0xf, 0xf, false);
+      t += __builtin_amdgcn_update_dpp(0, t, 0x114, 0xf, 0xf, false);
+      t += __builtin_amdgcn_update_dpp(0, t, 0x118, 0xf, 0xf, false);
+      run = t;
+      const int base = t - w.w;
+      const float v[4] = {alpha_fix<RULE>(base + w.x), alpha_fix<RULE>(base + w.y),
+                          alpha_fix<RULE>(base + w.z), alpha_fix<RULE>(base + w.w)};
+      if (in && c < M.W) MaskOut{out, 0}.put(c, 0, min(4, M.W - c), v);
     }
   }
 }
