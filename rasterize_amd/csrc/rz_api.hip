@@ -1567,6 +1567,9 @@ rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transf
   // no layer (the adjoint's own tile pass recomposites): the binned state only
   if (d_out) {
     dim3 fgrid((uint32_t)(ctx_x * cty));
+    const int split = rzk::scene_split(a.n_tiles, n, (uint32_t)ctx->n_cus);
+    const dim3 fblock(64 * split);
+    const uint32_t flds = (uint32_t)(split * ctx->cur.fine_lds);
     if (ctx->cur.scene_queue) {
       const size_t nt = (size_t)ctx_x * cty, nd = (size_t)(ctx_x + 1) * (cty + 1);
       RZ_TRY(ensure(ctx, ctx->sc_order, (nt + nd + 64) * 4));
@@ -1579,28 +1582,20 @@ rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transf
       a.order = ord;
       // persistent: as many waves as the chip holds of this kernel
       const uint32_t resident = (uint32_t)ctx->n_cus * 4u * (uint32_t)std::max(ctx->cur.scene_waves, 5);
-      fgrid = dim3(std::min<uint32_t>(a.n_tiles, resident));
+      fgrid = dim3(std::min<uint32_t>(a.n_tiles, resident / (uint32_t)split));
     }
     const int waves = ctx->cur.scene_waves;
-#define RZ_SCENE_FINE(W, Q)                                                                \
-  RZ_LAUNCH_LDS(ctx, "k_scene_fine", (rzk::k_scene_fine<W, Q, false>), fgrid, dim3(64),             \
-                ctx->cur.fine_lds, a, queue)
-    if (s->long_gradients) {
-      if (queue)
-        RZ_LAUNCH_LDS(ctx, "k_scene_fine", (rzk::k_scene_fine<1, true, true>), fgrid, dim3(64),
-                      ctx->cur.fine_lds, a, queue);
-      else
-        RZ_LAUNCH_LDS(ctx, "k_scene_fine", (rzk::k_scene_fine<1, false, true>), fgrid, dim3(64),
-                      ctx->cur.fine_lds, a, queue);
-    } else if (queue) {
-      if (waves == 8) RZ_SCENE_FINE(8, true);
-      else if (waves == 1) RZ_SCENE_FINE(1, true);
-      else RZ_SCENE_FINE(6, true);
-    } else {
-      if (waves == 8) RZ_SCENE_FINE(8, false);
-      else if (waves == 1) RZ_SCENE_FINE(1, false);
-      else RZ_SCENE_FINE(6, false);
-    }
+    using FineKernel = void (*)(rzk::SceneFineArgs, uint32_t*);
+#define RZ_SCENE_FINE(W, LONG)                                                             \
+  (split == 1 ? queue ? (FineKernel)rzk::k_scene_fine<W, true, LONG, 1>                    \
+                      : (FineKernel)rzk::k_scene_fine<W, false, LONG, 1>                   \
+   : queue    ? (FineKernel)rzk::k_scene_fine<W, true, LONG, rzk::kSplit>                  \
+              : (FineKernel)rzk::k_scene_fine<W, false, LONG, rzk::kSplit>)
+    const FineKernel fine = s->long_gradients ? RZ_SCENE_FINE(1, true)
+                            : waves == 8      ? RZ_SCENE_FINE(8, false)
+                            : waves == 1      ? RZ_SCENE_FINE(1, false)
+                                              : RZ_SCENE_FINE(6, false);
+    RZ_LAUNCH_LDS(ctx, "k_scene_fine", fine, fgrid, fblock, flds, a, queue);
 #undef RZ_SCENE_FINE
   } else {
     RZ_LAUNCH(ctx, "k_status_merge", rzk::k_status_merge, dim3(1), dim3(64), (const rzk::Status*)st,

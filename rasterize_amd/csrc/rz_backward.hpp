@@ -123,7 +123,7 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
   // forward sweep; a path with zero winding over the tile is skipped (the
   // reverse sweep writes its zero dL/dW)
   scene_paths(
-      a, L, TX, TY, lane, [](int, auto w) { return (float)w * (1.0f / kFix); },
+      a, L, TX, TY, 0u, nrow, lane, [](int, auto w) { return (float)w * (1.0f / kFix); },
       [&](const rzp::DPaint* paint, int rule, uint32_t, uint32_t t, int xs, int ys, bool,
           const float* W) {
         const rzp::DPaint p = load_const(paint);

@@ -1770,7 +1770,7 @@ template <int G>
 __device__ inline void tile_build(TileLDS<G>& L, const float4* recs, uint32_t rb, uint32_t re,
                                   const int4* events, uint32_t eb, uint32_t ee, int tx, int lane) {
   clear_tiles(L.acc[0], 1, lane);
-  __syncthreads();
+  wave_lds_sync();
   uint32_t rbs[G], pre[G + 1];
   pre[0] = 0;
 #pragma unroll
@@ -1780,7 +1780,7 @@ __device__ inline void tile_build(TileLDS<G>& L, const float4* recs, uint32_t rb
   }
   tile_records<G>(recs, rbs, pre, L, lane);
   tile_events(L.acc[0], events, eb, ee, tx, lane);
-  __syncthreads();
+  wave_lds_sync();
 }
 
 // A tile of any size, chunk by chunk, into the lanes' int64 sums in L.w64():
@@ -1803,7 +1803,7 @@ __device__ inline void tile_build_wide(TileLDS<G>& L, const float4* recs, uint32
     first = false;
     rb = r1;
     eb = e1;
-    __syncthreads();  // the next chunk clears the accumulators
+    wave_lds_sync();  // the next chunk clears the accumulators
   } while (rb < re || eb < ee);
 }
 

@@ -345,17 +345,17 @@ constexpr int kGroup = 4;
 // has no right-edge column, else int64), the first of them pixel (xs, ys) of
 // the path's sub-view; 0 outside the sub-view. flat: one value all over the
 // tile.
+// The paths are those of [begin, end) of the tile row's list.
 template <class Conv, class Px>
 __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, int TX, int TY,
-                                   int lane, Conv&& conv, Px&& px) {
-  const uint32_t nrow = a.row_count[TY];
+                                   uint32_t begin, uint32_t end, int lane, Conv&& conv, Px&& px) {
   const uint32_t* row = a.rows + (size_t)TY * a.n_paths;
-  for (uint32_t start = 0; start < nrow; start += 64) {
+  for (uint32_t start = begin; start < end; start += 64) {
     const uint32_t j = start + lane;
     uint32_t pid = 0, t = 0, rb = 0, re = 0, eb = 0, ee = 0;
     int bdv = 0;
     bool draw = false, right = false;
-    if (j < nrow) {
+    if (j < end) {
       pid = row[j];
       const int4 r = a.rects[pid];
       if (r.x <= TX && TX < r.z) {
@@ -403,7 +403,7 @@ __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, i
                                 lane_of(eb, src), lane_of(ee, src), TX - load_const(&a.pi[q].tx0), lane);
       } else if (l) {
         clear_tiles(L.acc[0], __popcll(l), lane);
-        __syncthreads();
+        wave_lds_sync();
         uint32_t rbs[kGroup], pre[kGroup + 1];
         pre[0] = 0;
         uint64_t lr = l;
@@ -423,7 +423,7 @@ __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, i
                         TX - load_const(&a.pi[lane_of(pid, src)].tx0), lane);
           }
         }
-        __syncthreads();
+        wave_lds_sync();
       }
       int k = 0;
       for (; g; g &= g - 1) {
@@ -472,7 +472,7 @@ __device__ inline void scene_paths(const SceneFineArgs& a, TileLDS<kGroup>& L, i
         }
         px(&P->paint, rule, q, qt, xs, ys, flat, v);
       }
-      __syncthreads();  // the accumulators are reused by the next group
+      wave_lds_sync();  // the accumulators are reused by the next group
     }
   }
 }
@@ -623,17 +623,27 @@ __device__ inline void blend_gradient(const rzp::DPaint& p, const GradLDS& G, in
   }
 }
 
-template <bool LONG>
-__device__ inline void scene_tile(const SceneFineArgs& a, TileLDS<kGroup>& L, uint32_t tile) {
-  const int lane = threadIdx.x;
+// One canvas tile by the workgroup's S waves: wave w composites its share of
+// the tile row's paths, the first wave over the background, the others over
+// nothing; source-over is associative, so wave 0 then composites the others'
+// results over its own, in order.
+template <bool LONG, int S>
+__device__ inline void scene_tile(const SceneFineArgs& a, TileLDS<kGroup>* Ls, uint32_t tile) {
+  const int lane = threadIdx.x & 63;
+  const int wave = S == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  TileLDS<kGroup>& L = Ls[wave];
   const int TX = (int)(tile % (uint32_t)a.tiles_x), TY = (int)(tile / (uint32_t)a.tiles_x);
   const int x = TX * 16 + lane_col(lane), y = TY * 16 + lane_row(lane);
   rzp::C4* out = a.out + (size_t)y * a.row_stride + x;
   rzp::C4 c[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) c[i] = a.load_dst && x + i < a.lw && y < a.lh ? out[i] : a.bg;
+  for (int i = 0; i < 4; ++i)
+    c[i] = wave ? rzp::splat(0.0f) : a.load_dst && x + i < a.lw && y < a.lh ? out[i] : a.bg;
+  const uint32_t nrow = load_const(a.row_count + TY);
+  const uint32_t share = (nrow + (uint32_t)S - 1u) / (uint32_t)S;
+  const uint32_t begin = min(nrow, share * (uint32_t)wave), end = min(nrow, begin + share);
   scene_paths(
-      a, L, TX, TY, lane,
+      a, L, TX, TY, begin, end, lane,
       [](int rule, auto w) { return rule == 0 ? alpha_fix<0>(w) : alpha_fix<1>(w); },
       [&](const rzp::DPaint* paint, int, uint32_t, uint32_t, int xs, int ys, bool flat,
           const float* alpha) {
@@ -676,36 +686,64 @@ __device__ inline void scene_tile(const SceneFineArgs& a, TileLDS<kGroup>& L, ui
           a2 = a3;
         }
       });
+  if (S > 1) {
+    rzp::C4* part = (rzp::C4*)L.acc;  // not in use any more: [i][lane]
+    static_assert(sizeof(L.acc) >= 4 * 64 * sizeof(rzp::C4), "a wave's colours fit its accumulators");
+    if (wave) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[i * 64 + lane] = c[i];
+    }
+    __syncthreads();
+    if (wave) return;
+    for (int w = 1; w < S; ++w) {
+      const rzp::C4* q = (const rzp::C4*)Ls[w].acc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c[i] = rzp::blend_over(c[i], q[i * 64 + lane]);
+    }
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     if (x + i < a.lw && y < a.lh) out[i] = c[i];
 }
 
-// One wave per workgroup. Without a queue (QUEUE false), workgroup i takes
-// canvas tile i. With one, the grid is persistent (a few waves per SIMD) and
-// each wave takes tiles from the front of a.order, costliest first, until
-// none is left: the tiles with the most paths start first instead of last.
-// The queue head comes as its own restrict parameter: the compiler then
-// knows its atomics touch nothing the tiles read, and the tiles' uniform
-// loads stay scalar.
+// Waves of a tile's workgroup. One wave takes a tile's paths one after the
+// other, which is the shortest time a frame can take however few tiles there
+// are; where the tiles leave the chip's 5,000 places for these waves idle
+// (five per SIMD, held there by their LDS), four waves share a tile's paths.
+// k_scene_fine of 240 shapes at 601x455 (1,102 tiles) 195 -> 176 us (what is
+// left is one tile with a path of thousands of records), of a tree of 49 fills
+// at 397x301 91 -> 64 us, of 16 paths at 256x256 30 -> 15 us.
+constexpr int kSplit = 4;
+inline int scene_split(uint32_t n_tiles, uint32_t n_paths, uint32_t n_cus) {
+  return n_tiles <= 8 * n_cus && n_paths >= 8 ? kSplit : 1;
+}
+
+// A workgroup of scene_split waves per canvas tile. Without a queue (QUEUE
+// false), workgroup i takes canvas tile i. With one, the grid is persistent (a
+// few waves per SIMD) and each workgroup takes tiles from the front of a.order,
+// costliest first, until none is left: the tiles with the most paths start
+// first instead of last. The queue head comes as its own restrict parameter:
+// the compiler then knows its atomics touch nothing the tiles read.
 // MINW: waves per SIMD the registers must allow (1: no bound; 6: 96 VGPRs,
 // for the five waves that LDS holds; 8: 80 VGPRs with some spilled). LONG: the
 // scene has a gradient that blend_gradient does not take (long_gradient).
-template <int MINW, bool QUEUE, bool LONG>
-__global__ __launch_bounds__(64, MINW == 6 ? 5 : MINW == 8 ? 6 : 1) void k_scene_fine(SceneFineArgs a,
-                                                         uint32_t* __restrict__ queue) {
-  __shared__ TileLDS<kGroup> L;
+// S: waves of a tile.
+template <int MINW, bool QUEUE, bool LONG, int S>
+__global__ __launch_bounds__(64 * S, MINW == 6 ? 5 : MINW == 8 ? 6 : 1) void k_scene_fine(
+    SceneFineArgs a, uint32_t* __restrict__ queue) {
+  __shared__ TileLDS<kGroup> L[S];
+  __shared__ uint32_t next;
   if (a.st->err || a.st->overflow) {
   } else if (!QUEUE) {
-    scene_tile<LONG>(a, L, blockIdx.x);
+    scene_tile<LONG, S>(a, L, blockIdx.x);
   } else {
     for (;;) {
-      uint32_t t = 0;
-      if (threadIdx.x == 0) t = atomicAdd(queue, 1u);
-      t = (uint32_t)__shfl((int)t, 0, 64);
+      if (threadIdx.x == 0) next = atomicAdd(queue, 1u);
+      __syncthreads();
+      const uint32_t t = next;
+      __syncthreads();  // `next` is read, the previous tile's LDS too
       if (t >= a.n_tiles) break;
-      __syncthreads();  // the previous tile's LDS reads are done
-      scene_tile<LONG>(a, L, a.order[t]);
+      scene_tile<LONG, S>(a, L, a.order[t]);
     }
   }
   // after the work: a global store ahead of the loads would keep the
