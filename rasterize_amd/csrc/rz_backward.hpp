@@ -240,49 +240,60 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
   }
 }
 
-// dL/dW of the path's pixel (x, y) of its sub-view, 0 outside the image.
-__device__ inline float gW_at(const PathInfo& P, const float* wbuf, int x, int y) {
-  if (x < 0 || y < 0 || x >= P.g.W || y >= P.g.H) return 0.0f;
-  const int gx = x + P.g.phx, gy = y + P.g.phy;
-  const uint32_t t = P.tile_base + (uint32_t)((gy >> 4) * P.g.tiles_x + (gx >> 4));
-  return wbuf[(size_t)t * 256 + (size_t)((gy & 15) * 16 + (gx & 15))];
-}
-
 // I0, I1 of one line (sub-view frame): for each pixel row it crosses and each
 // pixel column of that row, g_W times the exact integral of (1 - l) and l
-// over the y-range of the line inside the pixel.
-__device__ inline void line_integrals(const PathInfo& P, const float* wbuf, Pt a, Pt c, double* I0,
-                                      double* I1) {
+// over the y-range of the line inside the pixel. dxdy is the line's dx/dy
+// (dy != 0).
+//
+// Rows and columns are one loop over the line's pixels: the lanes of a wave
+// hold lines of different directions, and nested loops would take the longest
+// row of any lane once per row. The pixel's g_W is asked for before its
+// y-range is worked out, and the divisions (by dx and dy) are the line's, not
+// the pixel's. 8,192 cubics of about 1,000 px at 1024x1024: k_scene_bwd_lines
+// 473 -> 336 us.
+__device__ inline void line_integrals(const PathInfo& P, const float* wbuf, Pt a, Pt c, double dxdy,
+                                      double* I0, double* I1) {
   *I0 = *I1 = 0.0;
   const double dy = c.y - a.y;
-  if (dy == 0.0) return;
-  const double dxdy = (c.x - a.x) / dy;
   const double ylo = fmax(fmin(a.y, c.y), 0.0), yhi = fmin(fmax(a.y, c.y), (double)P.g.H);
   if (!(ylo < yhi)) return;
-  const int r0 = (int)floor(ylo), r1 = (int)ceil(yhi);
+  const double inv_dy = 1.0 / dy, dydx = 1.0 / dxdy;
+  // a line this steep stays in one column (or straddles x = 0, whose left
+  // side has no pixels): nothing to cut
+  const bool steep = !(fabs(dxdy) >= 1e-300);
+  const int r1 = (int)ceil(yhi);
   const double sgn = dy > 0.0 ? 1.0 : -1.0;
-  for (int r = r0; r < r1; ++r) {
-    const double ya = fmax(ylo, (double)r), yb = fmin(yhi, (double)r + 1.0);
-    if (!(ya < yb)) continue;
-    const double xa = a.x + (ya - a.y) * dxdy, xb = a.x + (yb - a.y) * dxdy;
-    const int cmin = max((int)floor(fmin(xa, xb)), 0);
-    const int cmax = min((int)floor(fmax(xa, xb)), P.g.W - 1);
-    for (int cx = cmin; cx <= cmax; ++cx) {
-      double lo = ya, hi = yb;
-      if (dxdy != 0.0) {
-        const double y0 = a.y + ((double)cx - a.x) / dxdy, y1 = a.y + ((double)cx + 1.0 - a.x) / dxdy;
-        lo = fmax(lo, fmin(y0, y1));
-        hi = fmin(hi, fmax(y0, y1));
-      }
-      if (!(lo < hi)) continue;
-      const float gw = gW_at(P, wbuf, cx, r);
-      if (gw == 0.0f) continue;
-      const double l0 = (lo - a.y) / dy, l1 = (hi - a.y) / dy;
-      const double len = sgn * (hi - lo);  // signed, in the line's direction
-      const double lm = 0.5 * (l0 + l1);
-      *I0 += (double)gw * len * (1.0 - lm);
-      *I1 += (double)gw * len * lm;
+  int r = (int)floor(ylo), cx = 0, ce = -1;
+  double ya = ylo, yb = ylo, xb = a.x + (ylo - a.y) * dxdy;
+  const float* row = nullptr;
+  --r;
+  while (true) {
+    if (cx > ce) {
+      if (++r >= r1) break;
+      const double xa = xb;
+      ya = yb;
+      yb = fmin(yhi, (double)r + 1.0);
+      xb = a.x + (yb - a.y) * dxdy;
+      cx = max((int)floor(fmin(xa, xb)), 0);
+      ce = min((int)floor(fmax(xa, xb)), P.g.W - 1);
+      const int gy = r + P.g.phy;
+      row = wbuf + (size_t)(P.tile_base + (uint32_t)((gy >> 4) * P.g.tiles_x)) * 256 + (gy & 15) * 16;
+      if (cx > ce) continue;
     }
+    const int gx = cx + P.g.phx;
+    const float gw = row[(size_t)(gx >> 4) * 256 + (gx & 15)];
+    double lo = ya, hi = yb;
+    if (!steep) {
+      const double y0 = a.y + ((double)cx - a.x) * dydx, y1 = a.y + ((double)cx + 1.0 - a.x) * dydx;
+      lo = fmax(lo, fmin(y0, y1));
+      hi = fmin(hi, fmax(y0, y1));
+    }
+    ++cx;
+    if (!(lo < hi)) continue;
+    const double len = sgn * (hi - lo);  // signed, in the line's direction
+    const double lm = 0.5 * ((lo - a.y) * inv_dy + (hi - a.y) * inv_dy);
+    *I0 += (double)gw * len * (1.0 - lm);
+    *I1 += (double)gw * len * lm;
   }
 }
 
@@ -331,10 +342,11 @@ __device__ void bwd_line_item(const DPath& p, uint32_t slot, uint32_t j, int D0,
 #pragma unroll
   for (int i = 0; i < NP; ++i) gp[i][0] = gp[i][1] = 0.0;
   auto on_leaf = [&](Pt a, Pt c, int depth, uint64_t bits) {
+    if (c.y == a.y) return;
     double I0, I1;
-    line_integrals(P, b.wbuf, a, c, &I0, &I1);
-    if (I0 == 0.0 && I1 == 0.0) return;
     const double s = (c.x - a.x) / (c.y - a.y);
+    line_integrals(P, b.wbuf, a, c, s, &I0, &I1);
+    if (I0 == 0.0 && I1 == 0.0) return;
     const double ga[2] = {-I0, s * I0}, gc[2] = {-I1, s * I1};
     const double scale = ldexp(1.0, -depth);
     double wa[NP], wc[NP];
