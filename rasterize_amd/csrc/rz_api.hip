@@ -527,8 +527,9 @@ struct Pack {
   std::vector<char> h;
   size_t put(const void* src, size_t bytes) {
     const size_t at = (h.size() + 15) & ~(size_t)15;
-    h.resize(at + std::max<size_t>(bytes, 1));
-    if (bytes) std::memcpy(h.data() + at, src, bytes);
+    h.resize(at);
+    if (bytes) h.insert(h.end(), (const char*)src, (const char*)src + bytes);
+    else h.push_back(0);
     return at;
   }
   template <typename T>
@@ -665,6 +666,10 @@ static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out)
   RZ_TRY(validate_path(ctx, p));
   rz_dpath* d = new rz_dpath();
   Pack pk;
+  // all that path_pack puts (a vector that grows copies a large path twice)
+  const size_t slots = (size_t)p->n_segments + p->n_subpaths;
+  pk.h.reserve(16 * (size_t)(p->n_segments ? p->point_offsets[p->n_segments] : 0) + 32 * (size_t)p->n_subpaths +
+               18 * slots + 16 * rzk::kBlock + 256);
   const PathAt at = path_pack(p, d, pk);
   void* base = nullptr;
   rz_status st = dev_alloc(ctx, d->allocs, pk.h.size(), &base);
