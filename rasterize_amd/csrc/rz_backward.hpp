@@ -110,8 +110,10 @@ __device__ inline float solid_da(rzp::C4 c, rzp::C4 g, float D) {
 // 256 paths of 32 cubics at 1024x1024: 3034 -> 1974 us. A solid paint, the
 // same for all pixels, has sweeps of its own that load only its colour and
 // rule and take g's inner product with it once a pixel (1117 -> 1041 us;
-// 16 paths of 8 cubics at 256x256 63 -> 48 us).
-__global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
+// 16 paths of 8 cubics at 256x256 63 -> 48 us). Each path is a chain of
+// dependent loads, so waves in flight count: unbounded, the kernel took 129
+// VGPRs and three waves per SIMD; 1041 -> 1002 us at four, 911 at five.
+__global__ __launch_bounds__(64, 5) void k_scene_bwd_tiles(BwdTileArgs b) {
   const SceneFineArgs& a = b.f;
   if (a.st->err || a.st->overflow) return;
   __shared__ TileLDS<kGroup> L;
@@ -284,7 +286,8 @@ __global__ __launch_bounds__(64) void k_scene_bwd_tiles(BwdTileArgs b) {
 // row of any lane once per row. The pixel's g_W is asked for before its
 // y-range is worked out, and the divisions (by dx and dy) are the line's, not
 // the pixel's. 8,192 cubics of about 1,000 px at 1024x1024: k_scene_bwd_lines
-// 473 -> 336 us.
+// 473 -> 336 us, and 312 at four waves per SIMD instead of three (138 VGPRs
+// unbounded).
 __device__ inline void line_integrals(const PathInfo& P, const float* wbuf, Pt a, Pt c, double dxdy,
                                       double* I0, double* I1) {
   *I0 = *I1 = 0.0;
@@ -450,7 +453,7 @@ __device__ inline void bwd_line_dispatch(const DPath& p, uint32_t slot, uint32_t
   bwd_line_item<NP>(p, slot, j, D0, active, x, fl, pi, slot_path, b, gtr);
 }
 
-__global__ __launch_bounds__(kBlock) void k_scene_bwd_lines(DPath p, Xform x, double fl, uint32_t bl,
+__global__ __launch_bounds__(kBlock, 4) void k_scene_bwd_lines(DPath p, Xform x, double fl, uint32_t bl,
                                                              uint32_t bq, int dq, int dc,
                                                              const PathInfo* pi,
                                                              const uint32_t* slot_path,
