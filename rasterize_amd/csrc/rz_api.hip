@@ -471,25 +471,33 @@ rz_status validate_path(rz_ctx* ctx, const rz_path* p) {
   return RZ_OK;
 }
 
-// Device memory that lives as long as the resident object it belongs to
-// (recorded in `allocs`), or, inside a TempScope, until the blocking call
-// returns.
-constexpr size_t kTempKeep = (size_t)256 << 20;  // bytes kept between blocking calls at most
-rz_status dev_alloc(rz_ctx* ctx, std::vector<void*>& allocs, size_t bytes, void** out) {
+// Device memory until the open TempScope ends: from the context's blocks.
+rz_status temp_alloc(rz_ctx* ctx, size_t bytes, void** out) {
   bytes = (std::max<size_t>(bytes, 16) + 255) & ~(size_t)255;
-  if (ctx->temp_open)
-    for (auto& b : ctx->temp)
-      if (b.cap - b.at >= bytes) {
-        *out = b.p + b.at;
-        b.at += bytes;
-        return RZ_OK;
-      }
-  const size_t want = ctx->temp_open ? std::max<size_t>(bytes, (size_t)4 << 20) : bytes;
+  for (auto& b : ctx->temp)
+    if (b.cap - b.at >= bytes) {
+      *out = b.p + b.at;
+      b.at += bytes;
+      return RZ_OK;
+    }
+  const size_t want = std::max<size_t>(bytes, (size_t)4 << 20);
   void* p = nullptr;
   hipError_t e = hipMalloc(&p, want);
   if (e != hipSuccess) return fail(ctx, RZ_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-  if (ctx->temp_open) ctx->temp.push_back({(char*)p, want, bytes});
-  else allocs.push_back(p);
+  ctx->temp.push_back({(char*)p, want, bytes});
+  *out = p;
+  return RZ_OK;
+}
+
+// Device memory that lives as long as the resident object it belongs to
+// (recorded in `allocs`), or, inside a TempScope, until that ends.
+constexpr size_t kTempKeep = (size_t)256 << 20;  // bytes kept between blocking calls at most
+rz_status dev_alloc(rz_ctx* ctx, std::vector<void*>& allocs, size_t bytes, void** out) {
+  if (ctx->temp_open) return temp_alloc(ctx, bytes, out);
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, std::max<size_t>(bytes, 16));
+  if (e != hipSuccess) return fail(ctx, RZ_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+  allocs.push_back(p);
   *out = p;
   return RZ_OK;
 }
@@ -2392,7 +2400,6 @@ struct TreeRender {
   const rz_paint* paints;
   int mode;
   double flatness;
-  std::vector<void*> allocs;            // none: the call's TempScope holds layers and masks
   std::vector<rz_dscene*> scenes;       // batches
   std::vector<rz_dpath*> dpaths;        // clip paths
   std::vector<int> batch;               // fills waiting for their layer
@@ -2408,7 +2415,8 @@ struct TreeRender {
       delete d;
     }
   }
-  rz_status alloc(size_t bytes, void** p) { return dev_alloc(ctx, allocs, bytes, p); }
+  // layers and masks: the attempt's TempScope holds them
+  rz_status alloc(size_t bytes, void** p) { return temp_alloc(ctx, bytes, p); }
   rz_status new_layer(const rzh::BBox& b, rzp::C4 fill, DLayer* L) {
     const double v[4] = {b.mn.x, b.mn.y, b.mx.x, b.mx.y};
     layer_of(v, &L->x, &L->y, &L->w, &L->h);
@@ -3760,9 +3768,11 @@ rz_status rz_render_tree(rz_ctx* ctx, const rz_path* const* paths, size_t n_path
   if (!rgba || cap_px < (size_t)lw * lh || !lw || !lh) return RZ_OK;
   const rzp::C4 c = bg ? rzp::c4(bg[0], bg[1], bg[2], bg[3]) : rzp::splat(0.0f);
   rz_status st = RZ_OK;
-  TempScope scope(ctx);
   for (int attempt = 0; attempt < kRuns; ++attempt) {
-    TreeRender R{ctx, &tb, paints, edge_mode, flatness, {}, {}, {}, {}};
+    // a scope per attempt: one that missed capacity gives its layers, masks
+    // and uploads back before the next takes its own
+    TempScope scope(ctx);
+    TreeRender R{ctx, &tb, paints, edge_mode, flatness, {}, {}, {}};
     DLayer L;
     st = R.new_layer(lb, c, &L);
     if (st == RZ_OK) st = R.render(root_id, L);

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import rasterize_amd as rz
-from rasterize_amd import FillRule, SignedDifferenceRasterizer, Transform
+from rasterize_amd import FillRule, LinColor, PathBuilder, Scene, SignedDifferenceRasterizer, Transform
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +74,53 @@ def test_plain_form_keeps_the_uploaded_points():
     ds.update_device(moved.data_ptr())
     assert not np.array_equal(render(ds, True), ref)
     assert np.array_equal(render(ds, False), ref)
+
+
+def test_a_tree_that_misses_capacity_takes_its_layers_once():
+    """A cold context's first rz_render_tree misses the line capacity and runs
+    again. It must then hold no more device memory than a context whose
+    buffers had their size before the call."""
+    import ctypes as C
+    w, h, n = 1600, 1200, 4000
+    rng = np.random.default_rng(7)
+    pb = PathBuilder().move_to((0.0, 0.0))
+    for _ in range(n):
+        pb.cubic_to(*[tuple(p) for p in rng.uniform(0, 1, (3, 2)) * (w, h)])
+    sheet = PathBuilder().move_to((0.0, 0.0)).line_to((w, 0.0)).line_to((w, h)).line_to((0.0, h)).close().build()
+    group = Scene(Scene.GROUP, children=[Scene.fill(sheet, LinColor(0.1, 0.2, 0.1, 0.5)),
+                                         Scene.fill(pb.close().build(), LinColor(0.2, 0.1, 0.0, 0.3))])
+    view = (0.0, 0.0, float(w), float(h))
+    layer = 16 * w * h  # the window's, and one for the group under the opacity
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    def context():
+        ctx = rz.Context(0)
+        SignedDifferenceRasterizer(ctx=ctx).mask_f32(sheet, Transform.new_scale(0.01, 0.01), 16, 16, 0)
+        return ctx
+    out = torch.zeros((h, w, 4), device="cuda")
+    taken, images = [], []
+    for warm in (True, False):
+        ctx = context()
+        before = free()
+        if warm:
+            ds = rz.DeviceScene(group, ctx)
+            for _ in range(6):
+                ds.render_device(I, view, out.data_ptr(), w)
+                try:
+                    ctx.sync()
+                    break
+                except rz.RzError as e:
+                    assert e.status == rz._abi.RZ_E_CAPACITY
+            ds.close()
+        images.append(group.with_opacity(0.5).render(SignedDifferenceRasterizer(ctx=ctx), I, view).image)
+        taken.append(before - free())
+        c = [C.c_size_t() for _ in range(3)]
+        ctx.check(rz._abi.lib().rz_last_counts(ctx.h, *[C.byref(v) for v in c]))
+        assert c[0].value > max(1 << 16, 16 * (n + 2))  # more lines than a cold context has room for
+        ctx.close()
+    print(f"taken warm {taken[0] >> 20} MB, cold {taken[1] >> 20} MB, a layer {layer >> 20} MB", flush=True)
+    assert np.array_equal(*images)
+    assert taken[1] < taken[0] + layer // 2
