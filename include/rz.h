@@ -289,7 +289,10 @@ rz_status rz_scene_free(rz_ctx* ctx, rz_dscene* scene);
  * RZ_EDGE_NONE: ActiveEdge). batched = 1 renders every path in one pipeline
  * (per-tile path lists, one store per pixel); batched = 0 runs the fill
  * pipeline once per path (the plain form). Asynchronous; errors at rz_sync.
- * The batched form has no reference counterpart. */
+ * (A set uploaded without paints and rules keeps no copy for the plain form:
+ * its first plain render uploads one and waits, and is refused with
+ * RZ_E_CAPACITY while the stream is being captured.) The batched form has no
+ * reference counterpart. */
 rz_status rz_render_device(rz_ctx* ctx, const rz_dscene* scene, rz_transform tr, double flatness,
                            int edge_mode, const double* view, const float* bg, int batched,
                            float* d_rgba, size_t row_stride);

@@ -220,6 +220,7 @@ struct rz_dpath {
   std::vector<void*> allocs;
   uint32_t n_order = 0;  // padded length of `order`
   uint32_t n_slots = 0;
+  std::vector<uint32_t> gaps;  // gap_slots
   bool has_bbox = false;  // Path::bbox(identity), for bounding-box paints
   SplitEst est;           // expected line counts of its quads / cubics
   rzh::BBox bbox{};
@@ -301,6 +302,12 @@ uint32_t blocks_for(size_t n) { return (uint32_t)((n + rzk::kBlock - 1) / rzk::k
 struct SplitSum {
   double q = 0, c = 0;  // sums of log counts
   size_t nq = 0, nc = 0;
+  void add(const SplitSum& o) {
+    q += o.q;
+    c += o.c;
+    nq += o.nq;
+    nc += o.nc;
+  }
   SplitEst est() const {
     SplitEst e;
     e.quad = nq ? std::exp(q / (double)nq) : 1.0;
@@ -571,7 +578,27 @@ struct PathAt {
   size_t pts, kinds, pt_off, slot_item, slot_flags, close_pts, order, gap_slots;
 };
 
-static PathAt path_pack(const rz_path* p, rz_dpath* d, Pack& pk) {
+// Appends a path's processing order: its slots grouped by kind, each group
+// padded to whole blocks.
+static void slot_order(const uint8_t* slot_kind, uint32_t n_slots, rz_dpath* d, std::vector<uint32_t>* order) {
+  const size_t first = order->size();
+  uint32_t nb[3] = {0, 0, 0};
+  for (int kind = 0; kind < 3; ++kind) {
+    const size_t before = order->size();
+    for (uint32_t t = 0; t < n_slots; ++t)
+      if (slot_kind[t] == kind) order->push_back(t);
+    nb[kind] = blocks_for(order->size() - before);
+    order->resize(before + (size_t)nb[kind] * rzk::kBlock, ~0u);
+  }
+  d->n_slots = d->view.n_slots = n_slots;
+  d->view.blocks_line = nb[0];
+  d->view.blocks_quad = nb[1];
+  d->view.blocks_cubic = nb[2];
+  d->n_order = (uint32_t)(order->size() - first);
+}
+
+// `sum`: the path's split_sum under the identity where the caller has it.
+static PathAt path_pack(const rz_path* p, rz_dpath* d, Pack& pk, const SplitSum* sum) {
   const uint32_t ns = p->n_segments, nsub = p->n_subpaths;
   const uint32_t npts = ns ? p->point_offsets[ns] : 0;
   const uint32_t nslots = ns + nsub;
@@ -622,17 +649,8 @@ static PathAt path_pack(const rz_path* p, rz_dpath* d, Pack& pk) {
   std::vector<uint32_t> gap_slots;
   for (uint32_t t = 0; t < nslots; ++t)
     if (slot_flags[t] & 1) gap_slots.push_back(t);
-  // processing order: kind-grouped, each group padded to whole blocks
   std::vector<uint32_t> order;
-  uint32_t nb[3] = {0, 0, 0};
-  for (int kind = 0; kind < 3; ++kind) {
-    size_t before = order.size();
-    for (uint32_t t = 0; t < nslots; ++t)
-      if (slot_kind[t] == kind) order.push_back(t);
-    size_t cnt = order.size() - before;
-    nb[kind] = blocks_for(cnt);
-    order.resize(before + (size_t)nb[kind] * rzk::kBlock, ~0u);
-  }
+  slot_order(slot_kind.data(), nslots, d, &order);
   PathAt at;
   at.pts = pk.put(p->points, 16 * (size_t)npts);
   at.kinds = pk.put(p->kinds, ns);
@@ -642,19 +660,13 @@ static PathAt path_pack(const rz_path* p, rz_dpath* d, Pack& pk) {
   at.close_pts = pk.put(close_pts);
   at.order = pk.put(order);
   at.gap_slots = pk.put(gap_slots);
-  rzk::DPath& v = d->view;
-  v.n_slots = nslots;
-  v.n_gaps = (uint32_t)gap_slots.size();
-  v.blocks_line = nb[0];
-  v.blocks_quad = nb[1];
-  v.blocks_cubic = nb[2];
-  d->n_order = (uint32_t)order.size();
-  d->n_slots = nslots;
+  d->view.n_gaps = (uint32_t)gap_slots.size();
+  d->gaps = std::move(gap_slots);
   const rzh::Tr ident = {{1.0, 0.0, 0.0, 0.0, 1.0, 0.0}};
   d->has_bbox = rzh::path_bbox(p, ident, &d->bbox);
-  SplitSum sum;
-  split_sum(p, ident.m, &sum);
-  d->est = sum.est();
+  SplitSum own;
+  if (!sum) split_sum(p, ident.m, &own);
+  d->est = (sum ? sum : &own)->est();
   return at;
 }
 
@@ -670,7 +682,8 @@ static void path_place(rz_dpath* d, const PathAt& at, const char* base) {
   v.gap_slots = (const uint32_t*)(base + at.gap_slots);
 }
 
-static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out) {
+static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out,
+                                  const SplitSum* sum = nullptr) {
   RZ_TRY(validate_path(ctx, p));
   rz_dpath* d = new rz_dpath();
   Pack pk;
@@ -678,7 +691,7 @@ static rz_status path_upload_impl(rz_ctx* ctx, const rz_path* p, rz_dpath** out)
   const size_t slots = (size_t)p->n_segments + p->n_subpaths;
   pk.h.reserve(16 * (size_t)(p->n_segments ? p->point_offsets[p->n_segments] : 0) + 32 * (size_t)p->n_subpaths +
                18 * slots + 16 * rzk::kBlock + 256);
-  const PathAt at = path_pack(p, d, pk);
+  const PathAt at = path_pack(p, d, pk, sum);
   void* base = nullptr;
   rz_status st = dev_alloc(ctx, d->allocs, pk.h.size(), &base);
   if (st == RZ_OK) st = pk.copy(ctx, base);
@@ -1185,8 +1198,7 @@ struct rz_dscene {
   uint64_t serial = g_serial.fetch_add(1);  // renewed by rz_atlas_set
   uint32_t n = 0;
   rz_dpath* all = nullptr;             // every path's segments, for the batched form
-  // one resident path each, for the plain form (made by its first render, in
-  // one block)
+  // one resident path each, for the plain form, in one block (ensure_per)
   mutable std::mutex per_mu;
   mutable std::vector<rz_dpath*> per;
   mutable std::vector<void*> per_allocs;
@@ -1231,6 +1243,7 @@ struct rz_dscene {
   struct HostRange {
     size_t seg, off, pt, sub, closed;
     uint32_t n_segments, n_subpaths;
+    SplitEst est;
   };
   std::vector<HostRange> host;
   std::vector<uint8_t> kinds, closed;
@@ -1313,6 +1326,7 @@ rz_status scene_upload_impl(rz_ctx* ctx, const rz_path* const* paths, const rz_p
   std::vector<int32_t> stop_user;
   std::vector<uint8_t> stop_flag;
   uint32_t user_stops = 0;
+  SplitSum sum;
   std::vector<size_t> stop_first(n);
   s->host_sp.resize(n);
   for (size_t i = 0; i < n; ++i) {
@@ -1325,7 +1339,11 @@ rz_status scene_upload_impl(rz_ctx* ctx, const rz_path* const* paths, const rz_p
     const rz_paint& paint_i = paints ? paints[i] : solid;
     const uint32_t seg0 = (uint32_t)kinds.size(), pt0 = (uint32_t)(pts.size() / 2);
     const uint32_t ns = p->n_segments, nsub = p->n_subpaths, npts = ns ? p->point_offsets[ns] : 0;
-    s->host.push_back({kinds.size(), s->offs.size(), pts.size(), s->subs.size(), closed.size(), ns, nsub});
+    SplitSum path_sum;
+    split_sum(p, rzh::Tr{{1.0, 0.0, 0.0, 0.0, 1.0, 0.0}}.m, &path_sum);
+    sum.add(path_sum);
+    s->host.push_back({kinds.size(), s->offs.size(), pts.size(), s->subs.size(), closed.size(), ns, nsub,
+                       path_sum.est()});
     if (ns) s->offs.insert(s->offs.end(), p->point_offsets, p->point_offsets + ns + 1);
     if (nsub) s->subs.insert(s->subs.end(), p->subpaths, p->subpaths + nsub + 1);
     for (uint32_t k = 0; k < ns; ++k) {
@@ -1374,7 +1392,7 @@ rz_status scene_upload_impl(rz_ctx* ctx, const rz_path* const* paths, const rz_p
   all.points = pts.data();
   all.subpaths = subs.data();
   all.closed = closed.data();
-  RZ_TRY(path_upload_impl(ctx, &all, &s->all));
+  RZ_TRY(path_upload_impl(ctx, &all, &s->all, &sum));
   // stops, then the ScenePath table pointing into them
   Pack pk;
   const size_t o_pos = pk.put(stop_pos), o_col = pk.put(stop_col), o_lin = pk.put(stop_lin);
@@ -1617,27 +1635,67 @@ rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transf
   return check_launch(ctx, "scene pass 1");
 }
 
-// The plain form's resident paths, all in one block. Scenes are drawn batched
-// unless the caller asks for the plain form, so its first render makes them.
+// The plain form's resident paths, all in one block. rz_scene_upload makes
+// them: the plain form is asynchronous, so it must find them. A glyph set (no
+// paints, no rules) is not meant to be drawn and holds none until someone does;
+// that render allocates and waits, which a capture of the stream cannot hold.
 rz_status ensure_per(rz_ctx* ctx, const rz_dscene* s) {
   std::lock_guard<std::mutex> lk(s->per_mu);
   if (!s->per.empty() || s->n == 0) return RZ_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  RZ_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
+  if (cap != hipStreamCaptureStatusNone)
+    return fail(ctx, RZ_E_CAPACITY, "a glyph set's first plain render while a frame is being captured");
+  // The batched form's tables serve here too (nothing writes them: a path's
+  // slots lie together and name the scene's segments and subpaths); its points
+  // do not (rz_scene_update_device). So a path adds its processing order.
+  const rz_dpath* all = s->all;
   std::vector<rz_dpath*> per(s->n);
-  std::vector<PathAt> at(s->n);
-  Pack pk;
+  std::vector<uint32_t> order, gaps;
+  std::vector<size_t> order_at(s->n), gaps_at(s->n);
+  std::vector<uint8_t> slot_kind;
+  uint32_t slot0 = 0;
+  size_t g = 0;
   for (uint32_t i = 0; i < s->n; ++i) {
     const rz_path hp = s->host_path(i);
-    per[i] = new rz_dpath();
-    at[i] = path_pack(&hp, per[i], pk);
+    rz_dpath* d = per[i] = new rz_dpath();
+    d->view = all->view;
+    slot_kind.clear();
+    for (uint32_t j = 0; j < hp.n_subpaths; ++j) {
+      slot_kind.insert(slot_kind.end(), hp.kinds + hp.subpaths[j], hp.kinds + hp.subpaths[j + 1]);
+      slot_kind.push_back(RZ_LINE);  // the closing line
+    }
+    const uint32_t n_slots = (uint32_t)slot_kind.size();
+    order_at[i] = order.size();
+    slot_order(slot_kind.data(), n_slots, d, &order);
+    gaps_at[i] = gaps.size();
+    for (; g < all->gaps.size() && all->gaps[g] < slot0 + n_slots; ++g) gaps.push_back(all->gaps[g] - slot0);
+    d->view.n_gaps = (uint32_t)(gaps.size() - gaps_at[i]);
+    d->view.slot_item += slot0;
+    d->view.slot_flags += slot0;
+    d->est = s->host[i].est;
+    slot0 += n_slots;
   }
+  const size_t pts_bytes = s->pts.size() * sizeof(double), order_bytes = order.size() * 4;
   void* base = nullptr;
-  rz_status st = dev_alloc(ctx, s->per_allocs, pk.h.size(), &base);
-  if (st == RZ_OK) st = pk.copy(ctx, base);
+  rz_status st = dev_alloc(ctx, s->per_allocs, pts_bytes + order_bytes + gaps.size() * 4, &base);
+  auto copy = [&](size_t at, const void* src, size_t bytes) -> rz_status {
+    if (bytes) RZ_HIP(ctx, hipMemcpyAsync((char*)base + at, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    return RZ_OK;
+  };
+  if (st == RZ_OK) st = copy(0, s->pts.data(), pts_bytes);
+  if (st == RZ_OK) st = copy(pts_bytes, order.data(), order_bytes);
+  if (st == RZ_OK) st = copy(pts_bytes + order_bytes, gaps.data(), gaps.size() * 4);
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess && st == RZ_OK) st = fail(ctx, RZ_E_HIP, "plain form upload");
   if (st != RZ_OK) {
     for (rz_dpath* d : per) delete d;
     return st;
   }
-  for (uint32_t i = 0; i < s->n; ++i) path_place(per[i], at[i], (const char*)base);
+  for (uint32_t i = 0; i < s->n; ++i) {
+    per[i]->view.pts = (const double*)base;
+    per[i]->view.order = (const uint32_t*)((char*)base + pts_bytes) + order_at[i];
+    per[i]->view.gap_slots = (const uint32_t*)((char*)base + pts_bytes + order_bytes) + gaps_at[i];
+  }
   s->per = std::move(per);
   return RZ_OK;
 }
@@ -3600,7 +3658,17 @@ rz_status rz_bin(rz_ctx* ctx, const rz_path* path, rz_transform tr, double flatn
 
 rz_status rz_scene_upload(rz_ctx* ctx, const rz_path* const* paths, const rz_paint* paints,
                           const int32_t* fill_rules, size_t n, rz_dscene** out) {
-  return scene_upload_impl(ctx, paths, paints, fill_rules, n, out);
+  rz_dscene* s = nullptr;
+  RZ_TRY(scene_upload_impl(ctx, paths, paints, fill_rules, n, out ? &s : nullptr));
+  if (paints || fill_rules) {
+    const rz_status st = ensure_per(ctx, s);
+    if (st != RZ_OK) {
+      (void)rz_scene_free(ctx, s);
+      return st;
+    }
+  }
+  *out = s;
+  return RZ_OK;
 }
 
 rz_status rz_scene_free(rz_ctx* ctx, rz_dscene* scene) {

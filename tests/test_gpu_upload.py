@@ -1,8 +1,8 @@
 """Device memory of blocking calls is taken from blocks the context keeps:
 results must not depend on what ran before, resident paths and scenes must not
-be touched by blocking calls in between, and the plain form's paths (made by
-its first render) must be the uploaded ones. Every comparison is bit for bit
-with the first run of the same call."""
+be touched by blocking calls in between, and the plain form's paths must be
+the uploaded ones and be there when rz_scene_upload returns. Every comparison
+is bit for bit with the first run of the same call."""
 import numpy as np
 import pytest
 import torch
@@ -74,6 +74,86 @@ def test_plain_form_keeps_the_uploaded_points():
     ds.update_device(moved.data_ptr())
     assert not np.array_equal(render(ds, True), ref)
     assert np.array_equal(render(ds, False), ref)
+
+
+class Hip:
+    """Capture of a context's stream through the HIP runtime torch has loaded."""
+
+    def __init__(self, ctx):
+        import ctypes as C
+        self.C, self.L = C, C.CDLL("libamdhip64.so")
+        self.stream = C.c_void_p(rz._abi.lib().rz_stream(ctx.h))
+
+    def check(self, s):
+        assert s == 0, s
+
+    def capture(self, call):
+        """call() captured and instantiated."""
+        C, L = self.C, self.L
+        self.check(L.hipStreamBeginCapture(self.stream, 0))
+        try:
+            call()
+        finally:
+            g = C.c_void_p()
+            s = L.hipStreamEndCapture(self.stream, C.byref(g))
+        self.check(s)
+        x = C.c_void_p()
+        self.check(L.hipGraphInstantiate(C.byref(x), g, None, None, C.c_size_t(0)))
+        return g, x
+
+    def launch(self, x):
+        self.check(self.L.hipGraphLaunch(x, self.stream))
+
+    def free(self, g, x):
+        self.check(self.L.hipGraphExecDestroy(x))
+        self.check(self.L.hipGraphDestroy(g))
+
+
+def test_the_first_plain_render_of_a_scene_can_be_captured():
+    """rz_render_device is asynchronous in both forms: with a context whose
+    buffers have their size, a scene's first plain render neither allocates nor
+    waits."""
+    w = h = 160
+    rng = np.random.default_rng(3)
+    fills = [(PathBuilder().move_to(tuple(rng.uniform(20, 140, 2))).circle(rng.uniform(5, 30)).build(),
+              LinColor(*(0.5 * rng.uniform(0, 1, 3)), 0.5)) for _ in range(12)]
+    scene = Scene(Scene.GROUP, children=[Scene.fill(*f) for f in fills])
+    view = (0.0, 0.0, float(w), float(h))
+    out = torch.zeros((h, w, 4), device="cuda")
+    torch.cuda.synchronize()
+    ctx = rz.Context(0)
+    warm = rz.DeviceScene(scene, ctx)
+    for _ in range(4):
+        warm.render_device(I, view, out.data_ptr(), w, batched=False)
+        try:
+            ctx.sync()
+            break
+        except rz.RzError as e:
+            assert e.status == rz._abi.RZ_E_CAPACITY
+    ref = out.cpu().numpy().copy()
+    hip = Hip(ctx)
+    fresh = rz.DeviceScene(scene, ctx)
+    g, x = hip.capture(lambda: fresh.render_device(I, view, out.data_ptr(), w, batched=False))
+    for k in range(3):
+        out.fill_(float(k))
+        torch.cuda.synchronize()
+        hip.launch(x)
+        ctx.sync()
+        assert np.array_equal(out.cpu().numpy(), ref), k
+        ctx.sync()
+    hip.free(g, x)
+    # a set without paints and rules keeps no copy: refused, and drawn once eager
+    paths = [f[0] for f in fills]
+    glyphs = rz.DeviceGlyphs(paths, [rz.atlas_slot(0, 0, 1, 1)] * len(paths), ctx)
+    bare = lambda: rz.DeviceScene.render_device(glyphs, I, view, out.data_ptr(), w, batched=False)  # noqa: E731
+    hip.check(hip.L.hipStreamBeginCapture(hip.stream, 0))
+    with pytest.raises(rz.RzError) as e:
+        bare()
+    gr = hip.C.c_void_p()
+    hip.check(hip.L.hipStreamEndCapture(hip.stream, hip.C.byref(gr)))
+    assert e.value.status == rz._abi.RZ_E_CAPACITY
+    bare()
+    ctx.sync()
 
 
 def test_a_tree_that_misses_capacity_takes_its_layers_once():
