@@ -1748,8 +1748,9 @@ rz_status enqueue_scene_plain(rz_ctx* ctx, const rz_dscene* s, const rz_transfor
 }
 
 // The glyphs of k_atlas_direct. Few glyphs go in one launch with the LDS of
-// the largest (two workgroups a CU hold them all at once); more in a launch per
-// size class (kDirectSmall).
+// the largest (the chip holds them all at once, or nearly: 500 of 132x135 px,
+// which run one a CU, 70 us, 125 by the pipeline); more in a launch per size
+// class (kDirectSmall).
 rz_status enqueue_atlas_direct(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, double fl,
                                float* d_atlas, size_t row_stride, rzk::Status* st) {
   rzk::DirectArgs a;
@@ -2044,18 +2045,30 @@ __global__ void k_set_colors(rzk::ScenePath* sp, const float* colors, uint32_t n
     sp[i].paint.color = rzp::c4(colors[4 * i], colors[4 * i + 1], colors[4 * i + 2], colors[4 * i + 3]);
 }
 
-// Whether a glyph's mask can be made by k_atlas_direct, and the largest
-// flatness bound and coordinate of its transformed curves. The accumulators
-// must fit (two workgroups a CU), the coordinates be finite, and the winding
-// stay in int32 at 2^-20: a flattened quad crosses a row at most twice, a
+// Whether a glyph's mask can be made by k_atlas_direct, the largest flatness
+// bound and coordinate of its transformed curves, and its straight segments.
+// The accumulators must fit, the coordinates be finite, and the winding stay
+// in int32 at 2^-20: a flattened quad crosses a row at most twice, a
 // cubic three times, a line once, which bounds any pixel's winding.
 struct DirectBound {
   double flatness = 0.0, coord = 0.0;
   bool cubics = false;
+  uint32_t n_lines = 0, n_long = 0;  // straight segments, the long ones (rzk::kDirectLong)
+  double long_px = 0.0;
 };
 bool direct_glyph(const rz_path* p, const rzk::AtlasSlot& a, DirectBound* out) {
   if (rzk::direct_lds((size_t)a.w, (size_t)a.h) > rzk::kDirectLds) return false;
   uint64_t crossings = p->n_subpaths;  // closing lines
+  auto straight = [&](const rzg::Pt& q, const rzg::Pt& r) {
+    const double len = std::fmax(std::fabs(r.x - q.x), std::fabs(r.y - q.y));
+    ++out->n_lines;
+    if (!(len > rzk::kDirectLong)) return;
+    ++out->n_long;
+    out->long_px += std::fmin(len, (double)(a.w + a.h));
+  };
+  auto point = [&](size_t k) { return rzg::tr_apply(a.m, rzg::mkpt(p->points[2 * k], p->points[2 * k + 1])); };
+  for (uint32_t j = 0; j < p->n_subpaths; ++j)
+    straight(point(p->point_offsets[p->subpaths[j + 1]] - 1), point(p->point_offsets[p->subpaths[j]]));
   for (uint32_t k = 0; k < p->n_segments; ++k) {
     const int np = p->kinds[k] + 2;
     crossings += p->kinds[k] + 1u;
@@ -2075,6 +2088,8 @@ bool direct_glyph(const rz_path* p, const rzk::AtlasSlot& a, DirectBound* out) {
     } else if (p->kinds[k] == RZ_CUBIC) {
       f = rzk::flatness_bound(n);
       out->cubics = true;
+    } else {
+      straight(n.p[0], n.p[1]);
     }
     out->flatness = std::max(out->flatness, f);
   }
@@ -2110,26 +2125,37 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
   if (t > 0xffffffffull || r > 0xffffffffull) return fail(ctx, RZ_E_ARG, "atlas too large");
   SplitSum sum;
   std::vector<uint32_t> slot_begin(s->n + 1), list;
+  rzk::DirectSet set;
   s->n_direct = s->n_binned = 0;
   s->direct_bound = s->direct_coord = 0.0;
   s->direct_cubics = false;
   for (uint32_t i = 0; i < s->n; ++i) {
     const rz_path hp = s->host_path(i);
-    split_sum(&hp, slots[i].tr.m, &sum);
+    SplitSum one;
+    split_sum(&hp, slots[i].tr.m, &one);
+    sum.add(one);
     slot_begin[i + 1] = slot_begin[i] + hp.n_segments + hp.n_subpaths;
     rzk::AtlasSlot& a = v[i];
     if (!a.w || !a.h) continue;
     DirectBound db;
     if (direct_glyph(&hp, a, &db)) {
-      a.direct = 1;
       list.push_back(i);
       s->direct_bound = std::max(s->direct_bound, db.flatness);
       s->direct_coord = std::max(s->direct_coord, db.coord);
       s->direct_cubics = s->direct_cubics || db.cubics;
+      const SplitEst e = one.est();
+      const double lines = db.n_lines + 1.4 * ((double)one.nq * e.quad + (double)one.nc * e.cubic);
+      const uint32_t n_slots = hp.n_segments + hp.n_subpaths;
+      set.add(rzk::direct_cost(a.w, a.h, n_slots, lines, db.n_long, db.long_px), n_slots);
     } else {
       ++s->n_binned;
     }
   }
+  if (!set.direct(s->n_binned)) {
+    s->n_binned += (uint32_t)list.size();
+    list.clear();
+  }
+  for (uint32_t i : list) v[i].direct = 1;
   s->n_direct = (uint32_t)list.size();
   // size classes, the largest first (and within a class the longest paths):
   // each is launched with the LDS of its largest glyph

@@ -3,6 +3,9 @@
 // LDS, without the binning stage. Used for the glyphs of an atlas whose masks
 // fit (direct_lds); larger ones go through the tile pipeline.
 #pragma once
+#include <algorithm>
+#include <cmath>
+
 #include "rz_scene.hpp"
 
 namespace rzk {
@@ -10,8 +13,19 @@ namespace rzk {
 constexpr int kDirectBlock = 512;  // threads at most (and at least kDirectSlots)
 constexpr int kDirectSlots = 128;  // slots staged at once
 constexpr int kDirectDepth = 10;   // subdivision depth at most (checked on the host)
-// LDS of the accumulators at most: two workgroups per CU
+
+// A workgroup's LDS beside its accumulators: the staged slots and the scans.
+struct DirectLDS {
+  double2 pts[kDirectSlots][4];  // control points under the glyph's transform
+  uint32_t pre[kDirectSlots + 1];
+  uint32_t kd[kDirectSlots];  // kind | depth << 8
+  uint32_t half_total, nodes2[2];
+  int marks[kDirectBlock / 64][64];
+};
+// LDS of the accumulators at most. Up to 70,640 bytes leave room for two
+// workgroups a CU; a larger one runs alone (direct_cost).
 constexpr size_t kDirectLds = 70 << 10;
+constexpr size_t kCuLds = 160 << 10;
 
 // Accumulators: H rows of direct_stride(W) ints, 2^-20 fixed point; four
 // columns are a 16-byte read, and the odd number of them keeps neighbouring
@@ -58,6 +72,63 @@ RZ_HD int leaf_depth(double bound, double fl) {
 inline bool direct_ok(double bound, double max_coord, double fl) {
   return leaf_depth(bound, fl) <= kDirectDepth && max_coord * 1e-14 < 1e-7 * sqrt(fl);
 }
+
+// What a glyph costs by this kernel and by the tile pipeline, in ns: of a full
+// chip's time (direct, tiles), and of its workgroup's, with nothing beside it
+// (chain). `lines`: what its curves and straight segments flatten into;
+// straight ones longer than kDirectLong pixels are n_long and long_px in all.
+//
+// Fitted to sets of 20 to 30,000 equal glyphs of 8 to 1,500 px and 6 to 900
+// segments. A workgroup costs 12 to 23 ns however little it does, or what
+// its accumulators keep from the CU (two a CU at 132x133 px, 83 ns; one at
+// 132x135, 150); a line little; but a long line takes all lanes for its rows,
+// one line after the other, and a long side leaves most lanes of the row sums
+// idle. Alone, a workgroup's time is its rounds of staged slots and nodes. The
+// pipeline's price is in tiles, lines, and the records of long lines.
+constexpr double kDirectLong = 16.0;
+struct DirectCost {
+  double direct = 0.0, tiles = 0.0, chain = 0.0;
+};
+inline DirectCost direct_cost(int w, int h, uint32_t n_slots, double lines, uint32_t n_long, double long_px) {
+  DirectCost c;
+  const size_t lds = direct_lds((size_t)w, (size_t)h), all = lds + sizeof(DirectLDS);
+  const double kb = (double)all / 1024.0;
+  double base = std::fmin(std::fmax(12.0, 0.25 * lines), 22.5);
+  if (lds > kDirectSmall) base = (8.0 + 0.55 * kb) * (2 * all > kCuLds ? 2.0 : 1.0);
+  c.direct = base + 0.015 * lines + (0.012 + 0.00018 * kb) * long_px + 0.15 * std::max(std::max(w, h) - 256, 0);
+  c.tiles = 2.0 + 0.6 * ((w + 15) / 16) * ((h + 15) / 16) + 0.07 * lines + 0.012 * long_px;
+  const double rounds = std::fmax((double)n_slots / kDirectSlots, lines / (4.0 * kDirectBlock));
+  c.chain = 5000.0 + rounds * (9000.0 + 110.0 * std::min(std::max(w, h), 256)) + 400.0 * n_long +
+            100.0 * std::max(w - 256, 0);
+  return c;
+}
+
+// Whether a set's glyphs that this kernel can mask take less time here than
+// with the others (n_binned of them) in the tile pipeline. The pipeline's
+// launches cost 60 us and its longest path some; where it runs anyway, it
+// still looks at every slot masked here. Measured, us here and there: 5,000
+// glyphs of 16x16 and 20 segments 116, 95, 1,000 of them 30, 57; 10,000 of
+// 48x48 of 20 225, 189, of 60 279, 336; 4,000 of 132x135 602, 454, 300 of
+// them 61, 106; 2,000 polygons of 100 lines in 100x100 236, 218, of 30 127,
+// 155; 2,000 of 1500x10 589, 286; 100 of 64x64 of 900 segments 126, 104, of 300
+// 51, 67; 400 of 60x60 with one of 200x200 103, 82, 4,000 with one 231, 289.
+constexpr double kTilesFixed = 60000.0, kTilesChain = 20.0, kTilesSlot = 0.13, kDirectFixed = 10000.0;
+struct DirectSet {
+  DirectCost sum;  // (chain: the longest)
+  double slots = 0.0, most_slots = 0.0;
+  void add(const DirectCost& c, uint32_t n_slots) {
+    sum.direct += c.direct;
+    sum.tiles += c.tiles;
+    sum.chain = std::fmax(sum.chain, c.chain);
+    slots += n_slots;
+    most_slots = std::fmax(most_slots, (double)n_slots);
+  }
+  bool direct(uint32_t n_binned) const {
+    const double here = kDirectFixed + std::fmax(sum.chain, sum.direct);
+    if (n_binned) return here + kTilesSlot * slots < sum.tiles;
+    return here < kTilesFixed + kTilesChain * most_slots + sum.tiles;
+  }
+};
 
 struct DirectArgs {
   DPath p;
@@ -282,13 +353,14 @@ template <int RULE, bool CUBIC>
 __global__ __launch_bounds__(kDirectBlock) void k_atlas_direct(DirectArgs a) {
   extern __shared__ int4 acc4[];
   int* acc = (int*)acc4;
-  __shared__ double2 pts[kDirectSlots][4];
-  __shared__ uint32_t pre[kDirectSlots + 1];
-  __shared__ uint32_t kd[kDirectSlots];  // kind | depth << 8
-  __shared__ uint32_t half_total, nodes2[2];
-  __shared__ int marks_all[kDirectBlock / 64][64];
+  __shared__ DirectLDS L;
+  auto& pts = L.pts;
+  auto& pre = L.pre;
+  auto& kd = L.kd;
+  auto& half_total = L.half_total;
+  auto& nodes2 = L.nodes2;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = (int)blockDim.x;
-  int* marks = marks_all[wave];
+  int* marks = L.marks[wave];
   const uint32_t glyph = load_const(a.list + blockIdx.x);
   const AtlasSlot S = load_const(a.slots + glyph);
   rzg::BinGrid g{};

@@ -124,3 +124,94 @@ def test_updated_points_and_not_a_number():
         rz.mask_atlas([a, bad], [rz.atlas_slot(0, 0, 60, 50), rz.atlas_slot(60, 0, 60, 50)],
                       np.zeros((50, 120), np.float32))
     assert e.value.status == rz._abi.RZ_E_NAN
+
+
+def route(paths, sizes, rule=FillRule.NonZero, mode=rz._abi.RZ_EDGE_MASK):
+    """Lines and records of one call over a set of glyphs in rows: glyphs of
+    k_atlas_direct make lines only."""
+    import ctypes as C
+    width = 4096
+    slots, x, y, row = [], 0, 0, 0
+    for w, h in sizes:
+        if x + w > width:
+            x, y, row = 0, y + row, 0
+        slots.append(rz.atlas_slot(x, y, w, h))
+        x, row = x + w, max(row, h)
+    ctx = rz.Context(0)
+    g = rz.DeviceGlyphs(paths, slots, ctx)
+    out = torch.zeros((y + row, width), device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(6):
+        g.mask_device(out.data_ptr(), width, fill_rule=rule, edge_mode=mode)
+        try:
+            ctx.sync()
+            break
+        except rz.RzError as e:
+            assert e.status == rz._abi.RZ_E_CAPACITY
+    c = [C.c_size_t() for _ in range(3)]
+    ctx.check(rz._abi.lib().rz_last_counts(ctx.h, *[C.byref(v) for v in c]))
+    atlas = out.cpu().numpy()
+    g.close()
+    ctx.close()
+    return c[0].value, c[1].value, atlas, slots
+
+
+def of(n, w, h, segs, kinds="q", seed=15):
+    """n glyphs of w x h (of a few different paths) and their sizes."""
+    rng = np.random.default_rng(seed)
+    some = [blob(rng, w, h, segs, kinds) for _ in range(min(n, 8))]
+    return [some[k % len(some)] for k in range(n)], [(w, h)] * n
+
+
+def lines(n, w, h, k, seed=16):
+    rng = np.random.default_rng(seed)
+    some = []
+    for _ in range(8):
+        p = rng.uniform(0, 1, (k, 2)) * (w, h)
+        pb = PathBuilder().move_to(tuple(p[0]))
+        for q in p[1:]:
+            pb.line_to(tuple(q))
+        some.append(pb.close().build())
+    return [some[j % 8] for j in range(n)], [(w, h)] * n
+
+
+@pytest.mark.parametrize("what,make,direct", [
+    ("few small glyphs", lambda: of(1000, 16, 16, 20), True),
+    ("many small glyphs", lambda: of(12000, 16, 16, 20), False),
+    ("half a CU's LDS and more, few", lambda: of(3, 132, 135, 40), True),
+    ("half a CU's LDS and more, many", lambda: of(4000, 132, 135, 40), False),
+    ("just below half a CU's LDS, many", lambda: of(3000, 132, 132, 40), True),
+    ("beyond the accumulators", lambda: of(3, 132, 137, 40), False),
+    ("few long lines", lambda: lines(100, 100, 100, 30), True),
+    ("many long lines", lambda: lines(100, 100, 100, 200), False),
+    ("few segments in few glyphs", lambda: of(20, 64, 64, 100, "lq"), True),
+    ("many segments in few glyphs", lambda: of(20, 64, 64, 900, "lq"), False),
+    ("many segments in many glyphs", lambda: of(1500, 64, 64, 400, "lq"), True),
+    ("long strips", lambda: lines(400, 1500, 10, 30), False),
+], ids=lambda v: v.replace(" ", "_").replace("'", "") if isinstance(v, str) else "")
+def test_route(what, make, direct):
+    """A set goes where direct_cost and DirectSet put it; either way the masks
+    are the oracle's (tile pipeline: coordinates within a 16 px tile are rounded
+    to 2^-20 in f32 and deposits to 2^-20, of up to 25 lines in a pixel: 5e-5)."""
+    paths, sizes = make()
+    n_lines, records, atlas, slots = route(paths, sizes)
+    assert n_lines and (records == 0) == direct, what
+    for p, s in list(zip(paths, slots))[:8]:
+        got = atlas[s.y:s.y + s.height, s.x:s.x + s.width]
+        d = np.abs(got - O.sd_mask(p, Transform.identity(), s.width, s.height, 0)).max()
+        assert d <= (BAR if direct else 5e-5), (what, d)
+
+
+def test_route_beside_larger_glyphs():
+    """One glyph too large for the workgroup's LDS: the others join it in the
+    tile pipeline, unless they are enough to pay for a launch of their own."""
+    big, size = of(1, 200, 200, 60)
+    alone = route(big, size)[1]
+    for n, direct in ((400, False), (6000, True)):
+        paths, sizes = of(n, 60, 60, 60)
+        n_lines, records, atlas, slots = route(paths + big, sizes + size)
+        assert (records == alone) == direct and records >= alone
+        for p, s in [(paths[0], slots[0]), (paths[n - 1], slots[n - 1]), (big[0], slots[n])]:
+            got = atlas[s.y:s.y + s.height, s.x:s.x + s.width]
+            d = np.abs(got - O.sd_mask(p, Transform.identity(), s.width, s.height, 0)).max()
+            assert d <= 5e-5, d
