@@ -429,7 +429,9 @@ typedef struct rz_atlas_slot {
 } rz_atlas_slot;
 
 /* Glyph sets are uploaded with rz_scene_upload (paints and fill_rules may be
- * NULL); rz_atlas_set places them (one slot per path, resident with the set). */
+ * NULL); rz_atlas_set places them (one slot per path, resident with the set).
+ * A call that fails leaves the placement there was; it is refused while the
+ * stream is being captured. */
 rz_status rz_atlas_set(rz_ctx* ctx, rz_dscene* glyphs, const rz_atlas_slot* slots);
 
 /* Asynchronous Rasterizer::mask of every glyph into its view of the device

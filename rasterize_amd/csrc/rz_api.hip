@@ -478,6 +478,13 @@ rz_status validate_path(rz_ctx* ctx, const rz_path* p) {
   return RZ_OK;
 }
 
+// Whether the context's stream is being captured, by whomever: no allocation,
+// copy from the host or wait then.
+bool captured(rz_ctx* ctx) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+}
+
 // Device memory until the open TempScope ends: from the context's blocks.
 rz_status temp_alloc(rz_ctx* ctx, size_t bytes, void** out) {
   bytes = (std::max<size_t>(bytes, 16) + 255) & ~(size_t)255;
@@ -1218,25 +1225,28 @@ struct rz_dscene {
   rzp::C4* stop_lin_dev = nullptr;
   int32_t* stop_user_dev = nullptr;   // -1: a gradient's default stop
   uint8_t* stop_flag_dev = nullptr;   // 1: its gradient interpolates linear colours
-  // glyph atlas placement (rz_atlas_set): device slots and slice totals
-  rzk::AtlasSlot* atlas_slots = nullptr;
-  uint32_t* atlas_tile_glyph = nullptr;  // glyph of each atlas tile
-  std::vector<void*> atlas_allocs;
-  SplitEst atlas_est;                    // line estimate under the slots' transforms
-  uint32_t atlas_tiles = 0, atlas_bands = 0, atlas_rows = 0;
-  bool atlas_ready = false;
-  // glyphs masked by k_atlas_direct: their indices by size class (device),
-  // and what flattening them at a call's threshold needs
-  struct DirectClass {
-    uint32_t first, count;
-    size_t lds;
+  // glyph atlas placement (rz_atlas_set)
+  struct Placement {
+    std::vector<void*> allocs;
+    rzk::AtlasSlot* slots = nullptr;  // device
+    uint32_t* tile_glyph = nullptr;   // glyph of each atlas tile (device)
+    SplitEst est;                     // line estimate under the slots' transforms
+    uint32_t tiles = 0, bands = 0, rows = 0;  // slice totals
+    // glyphs masked by k_atlas_direct: their indices by size class (device),
+    // and what flattening them at a call's threshold needs
+    struct DirectClass {
+      uint32_t first, count;
+      size_t lds;
+    };
+    std::vector<DirectClass> direct;
+    uint32_t n_direct = 0, n_binned = 0;  // glyphs with pixels: direct, and the others
+    const uint32_t* direct_list = nullptr;
+    const uint32_t* direct_slots = nullptr;  // [n + 1] first flatten slot of each glyph
+    double direct_bound = 0.0, direct_coord = 0.0;  // largest flatness bound and coordinate
+    bool direct_cubics = false;           // some of them have cubics
   };
-  std::vector<DirectClass> direct;
-  uint32_t n_direct = 0, n_binned = 0;   // glyphs with pixels: direct, and the others
-  const uint32_t* direct_list = nullptr;
-  const uint32_t* direct_slots = nullptr;  // [n + 1] first flatten slot of each glyph
-  double direct_bound = 0.0, direct_coord = 0.0;  // largest flatness bound and coordinate
-  bool direct_cubics = false;            // some of them have cubics
+  Placement at;
+  bool atlas_ready = false;
   bool points_updated = false;           // the device's points are not the host's any more
   // host copies of the paths, one after the other: for Path::bbox(tr) and the
   // resident paths of the plain form, and the atlas's line estimate
@@ -1276,13 +1286,11 @@ void scene_release(rz_dscene* s) {
   }
   for (void* p : s->allocs) (void)hipFree(p);
   for (void* p : s->per_allocs) (void)hipFree(p);
-  for (void* p : s->atlas_allocs) (void)hipFree(p);
-  s->atlas_slots = nullptr;
-  s->atlas_tile_glyph = nullptr;
+  for (void* p : s->at.allocs) (void)hipFree(p);
+  s->at = {};
   s->per.clear();
   s->allocs.clear();
   s->per_allocs.clear();
-  s->atlas_allocs.clear();
   s->all = nullptr;
 }
 
@@ -1443,8 +1451,8 @@ TuneKey scene_tune_key(const rz_dscene* s, const rz_transform& tr, double flatne
 }
 
 TuneKey atlas_tune_key(const rz_dscene* s, double flatness, int mode) {
-  return tune_key(2, mode, (size_t)s->atlas_tiles * 256, s->all ? s->all->n_slots : 0,
-                  s->atlas_est, 1.0, flatness);
+  return tune_key(2, mode, (size_t)s->at.tiles * 256, s->all ? s->all->n_slots : 0,
+                  s->at.est, 1.0, flatness);
 }
 
 rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transform& tr,
@@ -1642,9 +1650,7 @@ rz_status enqueue_scene_batched(rz_ctx* ctx, const rz_dscene* s, const rz_transf
 rz_status ensure_per(rz_ctx* ctx, const rz_dscene* s) {
   std::lock_guard<std::mutex> lk(s->per_mu);
   if (!s->per.empty() || s->n == 0) return RZ_OK;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  RZ_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
-  if (cap != hipStreamCaptureStatusNone)
+  if (captured(ctx))
     return fail(ctx, RZ_E_CAPACITY, "a glyph set's first plain render while a frame is being captured");
   // The batched form's tables serve here too (nothing writes them: a path's
   // slots lie together and name the scene's segments and subpaths); its points
@@ -1755,34 +1761,34 @@ rz_status enqueue_atlas_direct(rz_ctx* ctx, const rz_dscene* s, int rule, int mo
                                float* d_atlas, size_t row_stride, rzk::Status* st) {
   rzk::DirectArgs a;
   a.p = s->all->view;
-  a.slots = s->atlas_slots;
-  a.slot_begin = s->direct_slots;
+  a.slots = s->at.slots;
+  a.slot_begin = s->at.direct_slots;
   a.fl = fl;
   a.mode = mode;
   a.out = d_atlas;
   a.row_stride = row_stride;
   a.st = st;
   auto launch = [&](uint32_t first, uint32_t count, size_t lds, uint32_t threads) {
-    a.list = s->direct_list + first;
+    a.list = s->at.direct_list + first;
     const dim3 grid(count), block(threads);
     if (rule == RZ_NONZERO) {
-      if (s->direct_cubics)
+      if (s->at.direct_cubics)
         RZ_LAUNCH_LDS(ctx, "k_atlas_direct<0>", (rzk::k_atlas_direct<0, true>), grid, block, lds, a);
       else
         RZ_LAUNCH_LDS(ctx, "k_atlas_direct<0>", (rzk::k_atlas_direct<0, false>), grid, block, lds, a);
     } else {
-      if (s->direct_cubics)
+      if (s->at.direct_cubics)
         RZ_LAUNCH_LDS(ctx, "k_atlas_direct<1>", (rzk::k_atlas_direct<1, true>), grid, block, lds, a);
       else
         RZ_LAUNCH_LDS(ctx, "k_atlas_direct<1>", (rzk::k_atlas_direct<1, false>), grid, block, lds, a);
     }
   };
-  if (s->n_direct <= 2 * (uint32_t)ctx->n_cus) {
+  if (s->at.n_direct <= 2 * (uint32_t)ctx->n_cus) {
     size_t lds = 0;
-    for (const auto& c : s->direct) lds = std::max(lds, c.lds);
-    launch(0, s->n_direct, lds, rzk::kDirectBlock);
+    for (const auto& c : s->at.direct) lds = std::max(lds, c.lds);
+    launch(0, s->at.n_direct, lds, rzk::kDirectBlock);
   } else {
-    for (const auto& c : s->direct)
+    for (const auto& c : s->at.direct)
       launch(c.first, c.count, c.lds, c.lds <= rzk::kDirectSmall ? 128 : 256);
   }
   return check_launch(ctx, "k_atlas_direct");
@@ -1793,15 +1799,15 @@ rz_status enqueue_atlas_direct(rz_ctx* ctx, const rz_dscene* s, int rule, int mo
 rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, double flatness,
                         float* d_atlas, size_t row_stride) {
   const uint32_t n = s->n;
-  if (n == 0 || s->atlas_tiles == 0) return RZ_OK;
+  if (n == 0 || s->at.tiles == 0) return RZ_OK;
   select_params(ctx, atlas_tune_key(s, flatness, mode));
   const double fl = 16.0 * flatness * flatness;
   // small glyphs in one workgroup each; ActiveEdgeRasterizer's left edge
   // (rzg::ae_chain) needs the pipeline, and points replaced on the device may
   // be outside the bounds made from the host's
-  const bool direct = s->n_direct && mode != RZ_EDGE_NONE && !s->points_updated &&
-                      rzk::direct_ok(s->direct_bound, s->direct_coord, fl);
-  if (direct && s->n_binned == 0) {
+  const bool direct = s->at.n_direct && mode != RZ_EDGE_NONE && !s->points_updated &&
+                      rzk::direct_ok(s->at.direct_bound, s->at.direct_coord, fl);
+  if (direct && s->at.n_binned == 0) {
     RZ_TRY(ensure(ctx, ctx->meta, rzk::kStatusWords * 4));
     RZ_LAUNCH(ctx, "k_fill_u32", rzk::k_fill_u32, dim3(1), dim3(64), (uint32_t*)ctx->meta.p,
               (size_t)rzk::kStatusWords, 0u);
@@ -1823,7 +1829,7 @@ rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, dou
     ctx->ev_cap = 1 << 14;
     RZ_TRY(ensure(ctx, ctx->events, (size_t)ctx->ev_cap * 16));
   }
-  const uint32_t ct = s->atlas_tiles, cb = s->atlas_bands, cr = s->atlas_rows;
+  const uint32_t ct = s->at.tiles, cb = s->at.bands, cr = s->at.rows;
   const size_t sw = rzk::kStatusWords;
   const size_t ro = redge_words(sw + 2 * (size_t)ct + cb);
   const size_t meta_u32 = ro + 2 * (size_t)cr + rzk::kParts + 1 + rzk::kLineParts;
@@ -1845,12 +1851,12 @@ rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, dou
             dim3((uint32_t)std::min<size_t>(blocks_for(meta_u32), 4096)), dim3(rzk::kBlock), meta,
             meta_u32, 0u);
   RZ_LAUNCH(ctx, "k_atlas_setup", rzk::k_atlas_setup, dim3(blocks_for(n)), dim3(rzk::kBlock),
-            (const rzk::AtlasSlot*)s->atlas_slots, n, mode, direct, pi);
+            (const rzk::AtlasSlot*)s->at.slots, n, mode, direct, pi);
   rzk::Xform x{};
   rzk::LineBufs lb;
   uint32_t* bin_fill = meta + meta_u32 - (rzk::kParts + 1 + rzk::kLineParts);
   int dq, dc;
-  split_depths(ctx, s->atlas_est, 1.0, flatness, &dq, &dc);
+  split_depths(ctx, s->at.est, 1.0, flatness, &dq, &dc);
   const bool fused = ctx->cur.fused != 0;
   RZ_TRY(enqueue_flatten(ctx, d, x, fl, pi, s->slot_path, st, bin_fill + rzk::kParts + 1, dq, dc,
                          mode, 0.0, rzg::WrapClip{-1.0, 1.0, 0, 0}, &lb, !fused));
@@ -1881,7 +1887,7 @@ rz_status enqueue_atlas(rz_ctx* ctx, const rz_dscene* s, int rule, int mode, dou
   rzk::AtlasFineArgs a;
   RZ_TRY(ensure(ctx, ctx->atlas_tiles, (size_t)ct * sizeof(rzk::AtlasTile)));
   RZ_LAUNCH(ctx, "k_atlas_tiles", rzk::k_atlas_tiles, dim3(blocks_for(ct)), dim3(rzk::kBlock),
-            (const rzk::PathInfo*)pi, (const uint32_t*)s->atlas_tile_glyph, ct,
+            (const rzk::PathInfo*)pi, (const uint32_t*)s->at.tile_glyph, ct,
             (const uint32_t*)tile_off, (const uint32_t*)ev_off, (const int32_t*)bd,
             (rzk::AtlasTile*)ctx->atlas_tiles.p);
   a.tiles = (const rzk::AtlasTile*)ctx->atlas_tiles.p;
@@ -2099,6 +2105,7 @@ bool direct_glyph(const rz_path* p, const rzk::AtlasSlot& a, DirectBound* out) {
 rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) {
   if (!ctx || !s) return RZ_E_ARG;
   if (s->n && !slots) return fail(ctx, RZ_E_ARG, "slots is NULL");
+  if (captured(ctx)) return fail(ctx, RZ_E_HIP, "rz_atlas_set while the stream is being captured");
   std::vector<rzk::AtlasSlot> v(s->n);
   uint64_t t = 0, b = 0, r = 0;
   for (uint32_t i = 0; i < s->n; ++i) {
@@ -2126,9 +2133,7 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
   SplitSum sum;
   std::vector<uint32_t> slot_begin(s->n + 1), list;
   rzk::DirectSet set;
-  s->n_direct = s->n_binned = 0;
-  s->direct_bound = s->direct_coord = 0.0;
-  s->direct_cubics = false;
+  rz_dscene::Placement at;
   for (uint32_t i = 0; i < s->n; ++i) {
     const rz_path hp = s->host_path(i);
     SplitSum one;
@@ -2140,23 +2145,23 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
     DirectBound db;
     if (direct_glyph(&hp, a, &db)) {
       list.push_back(i);
-      s->direct_bound = std::max(s->direct_bound, db.flatness);
-      s->direct_coord = std::max(s->direct_coord, db.coord);
-      s->direct_cubics = s->direct_cubics || db.cubics;
+      at.direct_bound = std::max(at.direct_bound, db.flatness);
+      at.direct_coord = std::max(at.direct_coord, db.coord);
+      at.direct_cubics = at.direct_cubics || db.cubics;
       const SplitEst e = one.est();
       const double lines = db.n_lines + 1.4 * ((double)one.nq * e.quad + (double)one.nc * e.cubic);
       const uint32_t n_slots = hp.n_segments + hp.n_subpaths;
       set.add(rzk::direct_cost(a.w, a.h, n_slots, lines, db.n_long, db.long_px), n_slots);
     } else {
-      ++s->n_binned;
+      ++at.n_binned;
     }
   }
-  if (!set.direct(s->n_binned)) {
-    s->n_binned += (uint32_t)list.size();
+  if (!set.direct(at.n_binned)) {
+    at.n_binned += (uint32_t)list.size();
     list.clear();
   }
   for (uint32_t i : list) v[i].direct = 1;
-  s->n_direct = (uint32_t)list.size();
+  at.n_direct = (uint32_t)list.size();
   // size classes, the largest first (and within a class the longest paths):
   // each is launched with the LDS of its largest glyph
   auto lds_of = [&](uint32_t i) { return rzk::direct_lds((size_t)v[i].w, (size_t)v[i].h); };
@@ -2166,41 +2171,40 @@ rz_status atlas_set_impl(rz_ctx* ctx, rz_dscene* s, const rz_atlas_slot* slots) 
     if (cx != cy) return cx > cy;
     return slot_begin[x + 1] - slot_begin[x] > slot_begin[y + 1] - slot_begin[y];
   });
-  s->direct.clear();
-  for (uint32_t k = 0; k < s->n_direct; ++k) {
-    if (k == 0 || class_of(list[k]) != class_of(list[k - 1])) s->direct.push_back({k, 0, 0});
-    auto& c = s->direct.back();
+  for (uint32_t k = 0; k < at.n_direct; ++k) {
+    if (k == 0 || class_of(list[k]) != class_of(list[k - 1])) at.direct.push_back({k, 0, 0});
+    auto& c = at.direct.back();
     ++c.count;
     c.lds = std::max(c.lds, lds_of(list[k]));
   }
-  s->atlas_est = sum.est();
+  at.est = sum.est();
   std::vector<uint32_t> tile_glyph(t);
   for (uint32_t i = 0; i < s->n; ++i) {
     const uint64_t end = i + 1 < s->n ? v[i + 1].tile_base : t;
     for (uint64_t k = v[i].tile_base; k < end; ++k) tile_glyph[k] = i;
   }
-  if (!s->atlas_allocs.empty()) {
-    RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    for (void* p : s->atlas_allocs) RZ_HIP(ctx, hipFree(p));
-    s->atlas_allocs.clear();
-  }
-  s->atlas_slots = nullptr;
-  s->atlas_tile_glyph = nullptr;
   Pack pk;
   const size_t o_slots = pk.put(v), o_glyph = pk.put(tile_glyph);
   const size_t o_list = pk.put(list), o_begin = pk.put(slot_begin);
   void* base = nullptr;
-  RZ_TRY(dev_alloc(ctx, s->atlas_allocs, pk.h.size(), &base));
-  RZ_TRY(pk.copy(ctx, base));
-  s->atlas_slots = (rzk::AtlasSlot*)((char*)base + o_slots);
-  s->atlas_tile_glyph = (uint32_t*)((char*)base + o_glyph);
-  s->direct_list = (const uint32_t*)((char*)base + o_list);
-  s->direct_slots = (const uint32_t*)((char*)base + o_begin);
-  s->atlas_tiles = (uint32_t)t;
-  s->atlas_bands = (uint32_t)b;
-  s->atlas_rows = (uint32_t)r;
+  // the old placement stays whole until the new one is
+  RZ_TRY(dev_alloc(ctx, at.allocs, pk.h.size(), &base));
+  rz_status st = pk.copy(ctx, base);
+  if (st != RZ_OK) {
+    for (void* p : at.allocs) (void)hipFree(p);
+    return st;
+  }
+  at.slots = (rzk::AtlasSlot*)((char*)base + o_slots);
+  at.tile_glyph = (uint32_t*)((char*)base + o_glyph);
+  at.direct_list = (const uint32_t*)((char*)base + o_list);
+  at.direct_slots = (const uint32_t*)((char*)base + o_begin);
+  at.tiles = (uint32_t)t;
+  at.bands = (uint32_t)b;
+  at.rows = (uint32_t)r;
+  std::swap(s->at, at);
   s->atlas_ready = true;
   s->serial = g_serial.fetch_add(1);  // frames captured with the old placement do not match
+  for (void* p : at.allocs) RZ_HIP(ctx, hipFree(p));  // (the copy waited for the calls that read it)
   return RZ_OK;
 }
 
@@ -2986,7 +2990,7 @@ rz_status rz_tune_atlas_device(rz_ctx* ctx, const rz_dscene* glyphs, double flat
   if (!glyphs || !glyphs->atlas_ready) return fail(ctx, RZ_E_ARG, "glyph placement not set");
   if (!d_atlas) return fail(ctx, RZ_E_ARG, "d_atlas is NULL");
   int adq, adc;
-  auto_depths(glyphs->atlas_est, 1.0, flatness, &adq, &adc);
+  auto_depths(glyphs->at.est, 1.0, flatness, &adq, &adc);
   return tune_search(ctx, atlas_tune_key(glyphs, flatness, edge_mode), adq, adc,
                      [&]() {
                        return enqueue_atlas(ctx, glyphs, fill_rule, edge_mode, flatness, d_atlas,
@@ -3944,7 +3948,7 @@ rz_status rz_scene_update_device(rz_ctx* ctx, rz_dscene* scene, const double* d_
     // the glyphs' bounds were made from the host's points: no k_atlas_direct
     // from now on, nor a frame captured with it
     scene->points_updated = true;
-    if (scene->n_direct) scene->serial = g_serial.fetch_add(1);
+    if (scene->at.n_direct) scene->serial = g_serial.fetch_add(1);
   }
   if (d_points && scene->n_points)
     RZ_HIP(ctx, hipMemcpyAsync((void*)scene->all->view.pts, d_points,

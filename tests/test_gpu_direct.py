@@ -215,3 +215,41 @@ def test_route_beside_larger_glyphs():
             got = atlas[s.y:s.y + s.height, s.x:s.x + s.width]
             d = np.abs(got - O.sd_mask(p, Transform.identity(), s.width, s.height, 0)).max()
             assert d <= 5e-5, d
+
+
+def test_a_placement_that_fails_leaves_the_one_before():
+    """rz_atlas_set that cannot be done (here: while its stream is being
+    captured) must leave the set as it was: the masks are those of the first
+    placement, bit for bit."""
+    import ctypes as C
+    from test_gpu_upload import Hip
+    paths, sizes = of(40, 60, 60, 30)
+    ctx = rz.Context(0)
+    small = [rz.atlas_slot(64 * k, 0, 60, 60) for k in range(40)]
+    g = rz.DeviceGlyphs(paths, small, ctx)
+    out = torch.zeros((512, 64 * 40), device="cuda")
+    torch.cuda.synchronize()
+
+    def run():
+        out.fill_(-1.0)
+        torch.cuda.synchronize()
+        for _ in range(4):
+            g.mask_device(out.data_ptr(), 64 * 40)
+            try:
+                ctx.sync()
+                return out.cpu().numpy().copy()
+            except rz.RzError as e:
+                assert e.status == rz._abi.RZ_E_CAPACITY
+    ref = run()
+    hip = Hip(ctx)
+    # the second placement: larger views, and some beyond the accumulators
+    large = (rz._abi.rz_atlas_slot * 40)(*[rz.atlas_slot(64 * k, 0, 60, 500 if k % 2 else 100) for k in range(40)])
+    hip.check(hip.L.hipStreamBeginCapture(hip.stream, 0))
+    s = rz._abi.lib().rz_atlas_set(ctx.h, g.h, large)
+    graph = C.c_void_p()
+    hip.check(hip.L.hipStreamEndCapture(hip.stream, C.byref(graph)))
+    assert s == rz._abi.RZ_E_HIP
+    assert np.array_equal(run(), ref)
+    ctx.check(rz._abi.lib().rz_atlas_set(ctx.h, g.h, large))
+    again = run()
+    assert not np.array_equal(again, ref) and (again[:100, :60] >= 0.0).all()
