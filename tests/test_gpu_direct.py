@@ -1,6 +1,7 @@
-"""Glyphs masked in one workgroup (k_atlas_direct) against the oracle: mask
-sizes around 16-pixel columns, one pixel, and the largest the accumulators
-hold, next to glyphs that go through the tile pipeline (too large, too many
+"""Glyphs masked in one workgroup (k_atlas_direct) and through the tile
+pipeline, and which of the two a set takes (rz_atlas_set), against the oracle:
+mask sizes around 16-pixel columns, one pixel, and the largest the accumulators
+hold, next to glyphs that need the tile pipeline (too large, too many
 segments), with lines, quads and cubics, long edges, paths crossing every side
 of their view, both edge modes and fill rules, more slots than are staged at
 once, and a flatness that needs the deepest subdivision.
@@ -41,7 +42,7 @@ def blob(rng, w, h, n, kinds="lqc", over=0.0):
     return pb.close().build()
 
 
-def check(paths, sizes, rule, mode, trs=None, flatness=0.05):
+def check(paths, sizes, rule, mode, trs=None, flatness=0.05, direct=None):
     trs = trs or [Transform.identity()] * len(paths)
     slots, x = [], 3
     for (w, h), tr in zip(sizes, trs):
@@ -50,6 +51,8 @@ def check(paths, sizes, rule, mode, trs=None, flatness=0.05):
     atlas = np.full((max(h for _, h in sizes) + 5, x + 4), -1.0, np.float32)
     inside = np.zeros(atlas.shape, bool)
     rz.mask_atlas(paths, slots, atlas, rule, flatness=flatness, edge_mode=mode)
+    if direct is not None:  # glyphs of k_atlas_direct make no records
+        assert (last_counts(rz.default_context())[1] == 0) == direct
     worst = 0.0
     for p, s, tr in zip(paths, slots, trs):
         f = O.sd_mask if mode == rz._abi.RZ_EDGE_MASK else O.sd_mask_iter
@@ -74,6 +77,24 @@ def test_sizes_and_sides(rule, mode):
     check(paths, sizes, rule, mode)
 
 
+@pytest.mark.parametrize("rule", [FillRule.NonZero, FillRule.EvenOdd])
+@pytest.mark.parametrize("mode", [rz._abi.RZ_EDGE_MASK, rz._abi.RZ_EDGE_ITER])
+def test_sizes_and_sides_in_one_workgroup(rule, mode):
+    """The same without the glyphs that need the tile pipeline, which take the
+    small set with them; and long edges under transforms."""
+    rng = np.random.default_rng(11)
+    sizes = [(1, 1), (2, 5), (15, 16), (16, 17), (17, 33), (31, 1), (64, 64), (65, 3), (128, 128), (132, 135),
+             (40, 300), (270, 50)]
+    paths = [blob(rng, w, h, int(n), over=o) for (w, h), n, o in
+             zip(sizes, [3, 4, 9, 20, 127, 5, 129, 12, 200, 60, 7, 30], [0, .3, 0, .2, .1, .5, 0, .4, .05, .3, 0, .2])]
+    check(paths, sizes, rule, mode, direct=True)
+    sizes = [(96, 120), (50, 40), (100, 90)]
+    paths = [blob(rng, 96, 120, 4, "l", 2.0), blob(rng, 50, 40, 6, "c", 3.0), blob(rng, 100, 90, 30)]
+    trs = [Transform.identity(), Transform.new_rotate(0.4),
+           Transform.new_translate(20.0, -15.0) * Transform.new_scale(1.7, 0.6)]
+    check(paths, sizes, rule, mode, trs, direct=True)
+
+
 def test_transforms_long_edges_and_many_segments():
     rng = np.random.default_rng(12)
     sizes = [(96, 120), (50, 40), (60, 60), (100, 90)]
@@ -90,7 +111,7 @@ def test_transforms_long_edges_and_many_segments():
 def test_flatness(flatness):
     rng = np.random.default_rng(13)
     check([blob(rng, 60, 50, 12), blob(rng, 30, 30, 5, "qc", 0.5)], [(60, 50), (30, 30)], FillRule.NonZero,
-          rz._abi.RZ_EDGE_MASK, flatness=flatness)
+          rz._abi.RZ_EDGE_MASK, flatness=flatness, direct=True)
 
 
 def test_updated_points_and_not_a_number():
@@ -126,10 +147,16 @@ def test_updated_points_and_not_a_number():
     assert e.value.status == rz._abi.RZ_E_NAN
 
 
-def route(paths, sizes, rule=FillRule.NonZero, mode=rz._abi.RZ_EDGE_MASK):
+def last_counts(ctx):
+    import ctypes as C
+    c = [C.c_size_t() for _ in range(3)]
+    ctx.check(rz._abi.lib().rz_last_counts(ctx.h, *[C.byref(v) for v in c]))
+    return [v.value for v in c]
+
+
+def route(paths, sizes, rule=FillRule.NonZero, mode=rz._abi.RZ_EDGE_MASK, flatness=0.05):
     """Lines and records of one call over a set of glyphs in rows: glyphs of
     k_atlas_direct make lines only."""
-    import ctypes as C
     width = 4096
     slots, x, y, row = [], 0, 0, 0
     for w, h in sizes:
@@ -142,18 +169,17 @@ def route(paths, sizes, rule=FillRule.NonZero, mode=rz._abi.RZ_EDGE_MASK):
     out = torch.zeros((y + row, width), device="cuda")
     torch.cuda.synchronize()
     for _ in range(6):
-        g.mask_device(out.data_ptr(), width, fill_rule=rule, edge_mode=mode)
+        g.mask_device(out.data_ptr(), width, fill_rule=rule, flatness=flatness, edge_mode=mode)
         try:
             ctx.sync()
             break
         except rz.RzError as e:
             assert e.status == rz._abi.RZ_E_CAPACITY
-    c = [C.c_size_t() for _ in range(3)]
-    ctx.check(rz._abi.lib().rz_last_counts(ctx.h, *[C.byref(v) for v in c]))
+    n_lines, records, _ = last_counts(ctx)
     atlas = out.cpu().numpy()
     g.close()
     ctx.close()
-    return c[0].value, c[1].value, atlas, slots
+    return n_lines, records, atlas, slots
 
 
 def of(n, w, h, segs, kinds="q", seed=15):
@@ -215,6 +241,56 @@ def test_route_beside_larger_glyphs():
             got = atlas[s.y:s.y + s.height, s.x:s.x + s.width]
             d = np.abs(got - O.sd_mask(p, Transform.identity(), s.width, s.height, 0)).max()
             assert d <= 5e-5, d
+
+
+@pytest.mark.parametrize("rule", [FillRule.NonZero, FillRule.EvenOdd])
+@pytest.mark.parametrize("mode", [rz._abi.RZ_EDGE_MASK, rz._abi.RZ_EDGE_ITER])
+@pytest.mark.parametrize("oversized", [0, 3])
+def test_both_size_classes(rule, mode, oversized):
+    """More glyphs than one launch takes: a launch of two waves a glyph for the
+    small ones and of four for the others, of lines, quads and cubics, and the
+    same beside glyphs that need the tile pipeline."""
+    rng = np.random.default_rng(17)
+    some = []
+    for k in range(64):
+        w, h = rng.integers(20, 77, 2) if k % 2 else rng.integers(80, 129, 2)
+        some.append((blob(rng, w, h, int(rng.integers(30, 140)), ("q", "lqc", "c", "lq")[k % 4], over=(0.0, 0.3)[k % 3 == 0]),
+                     (int(w), int(h))))
+    big = [(blob(rng, 150, 160, 50), (150, 160)) for _ in range(oversized)]
+    glyphs = [some[k % 64] for k in range(2400)] + big
+    n_lines, records, atlas, slots = route([g[0] for g in glyphs], [g[1] for g in glyphs], rule, mode)
+    assert n_lines and (records == 0) == (oversized == 0)
+    if oversized:
+        assert records == route([g[0] for g in big], [g[1] for g in big], rule, mode)[1]
+    f = O.sd_mask if mode == rz._abi.RZ_EDGE_MASK else O.sd_mask_iter
+    refs = [f(p, Transform.identity(), w, h, rule, 0.05) for p, (w, h) in some + big]
+    worst = 0.0
+    for k, s in enumerate(slots):
+        direct = k < 2400
+        ref = refs[k % 64] if direct else refs[64 + k - 2400]
+        d = np.abs(atlas[s.y:s.y + s.height, s.x:s.x + s.width] - ref).max()
+        worst = max(worst, d)
+        assert d <= (BAR if direct else 5e-5), (k, s.width, s.height, d)
+    print(f"rule {rule}, mode {mode}, {oversized} oversized: max|d|={worst:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("mode", [rz._abi.RZ_EDGE_MASK, rz._abi.RZ_EDGE_NONE])
+def test_sets_of_the_tile_pipeline(mode):
+    """A set of glyphs beyond the accumulators, and small ones under
+    ActiveEdgeRasterizer, both of more lines than a cold context has room for
+    (the first run misses capacity). Bars as in test_gpu_mask.py."""
+    rng = np.random.default_rng(18)
+    side, n, flatness = (150, 300, 0.005) if mode == rz._abi.RZ_EDGE_MASK else (40, 900, 0.005)
+    some = [blob(rng, side, side, 30, "c", 0.1) for _ in range(10)]
+    for rule in (FillRule.NonZero, FillRule.EvenOdd):
+        n_lines, records, atlas, slots = route([some[k % 10] for k in range(n)], [(side, side)] * n, rule, mode,
+                                               flatness)
+        assert n_lines > max(1 << 16, 16 * n * 31) and records
+        f = O.sd_mask if mode == rz._abi.RZ_EDGE_MASK else O.ae_mask
+        refs = [f(p, Transform.identity(), side, side, rule, flatness) for p in some]
+        for k, s in enumerate(slots):
+            d = np.abs(atlas[s.y:s.y + s.height, s.x:s.x + s.width] - refs[k % 10])
+            assert d.max() <= 2e-3 and d.mean() <= 1e-5, (k, d.max())
 
 
 def test_a_placement_that_fails_leaves_the_one_before():
