@@ -13,7 +13,8 @@
  *     thread-safe: use one per host thread (the reference's rasterizers are
  *     `&self` and single-threaded).
  *   - Blocking entry points take host buffers and return when the result is
- *     in them. `_device` entry points take device pointers, are asynchronous
+ *     in them. Their copies on the device go into blocks of which the context
+ *     keeps up to 256 MiB for the next call, until rz_ctx_destroy. `_device` entry points take device pointers, are asynchronous
  *     on the context's stream and report errors at the next rz_sync(): the
  *     status of every call queued since the previous sync is merged (first
  *     error, every capacity miss), so RZ_E_CAPACITY there means the queued
@@ -470,7 +471,8 @@ rz_status rz_mask_atlas(rz_ctx* ctx, const rz_path* const* paths, const rz_atlas
  * 15): the scatter's grid holds at most 2^value waves. RZ_PARAM_SCENE_WAVES
  * (1, 6 or 8, default 6): the register budget of the batched scene's fine
  * kernel (1: unbounded; 6: 96 VGPRs, for the five waves per SIMD its LDS
- * allows; 8: 80 VGPRs). RZ_PARAM_SCENE_QUEUE (0 or 1,
+ * allows; 8: 80 VGPRs, as 1 where four waves share a tile: views of up to 8
+ * tiles a CU with 8 paths or more). RZ_PARAM_SCENE_QUEUE (0 or 1,
  * default 0): the batched scene's fine stage as a persistent grid taking
  * canvas tiles from a device queue, the tiles covered by the most paths
  * first. RZ_PARAM_FUSED (0 or 1, default 0): flatten and the binning's

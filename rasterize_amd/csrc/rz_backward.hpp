@@ -112,7 +112,10 @@ __device__ inline float solid_da(rzp::C4 c, rzp::C4 g, float D) {
 // rule and take g's inner product with it once a pixel (1117 -> 1041 us;
 // 16 paths of 8 cubics at 256x256 63 -> 48 us). Each path is a chain of
 // dependent loads, so waves in flight count: unbounded, the kernel took 129
-// VGPRs and three waves per SIMD; 1041 -> 1002 us at four, 911 at five.
+// VGPRs and three waves per SIMD; 1041 -> 1002 us at four, 911 at five, which
+// spill 39 registers where gradients are painted (240 shapes, two in five of
+// them gradients with stop gradients: 7,486 us, 7,766 before all of this; the
+// stops' atomics bound those).
 __global__ __launch_bounds__(64, 5) void k_scene_bwd_tiles(BwdTileArgs b) {
   const SceneFineArgs& a = b.f;
   if (a.st->err || a.st->overflow) return;
@@ -286,8 +289,8 @@ __global__ __launch_bounds__(64, 5) void k_scene_bwd_tiles(BwdTileArgs b) {
 // row of any lane once per row. The pixel's g_W is asked for before its
 // y-range is worked out, and the divisions (by dx and dy) are the line's, not
 // the pixel's. 8,192 cubics of about 1,000 px at 1024x1024: k_scene_bwd_lines
-// 473 -> 336 us, and 312 at four waves per SIMD instead of three (138 VGPRs
-// unbounded).
+// 473 -> 336 us, and 312 at four waves per SIMD (20 of 138 VGPRs spilled)
+// instead of three.
 __device__ inline void line_integrals(const PathInfo& P, const float* wbuf, Pt a, Pt c, double dxdy,
                                       double* I0, double* I1) {
   *I0 = *I1 = 0.0;

@@ -268,8 +268,11 @@ __device__ inline void direct_short(const DirectMask& M, const DirectPiece& q) {
   const int Y0 = fix_height(q.y0 - yr), Y1 = fix_height(q.y1 - yr);
   const int c0 = (int)xl;
   constexpr int one = 1 << rzg::kFixShift;
-  // per 2^-20 of a row; over at most four rows the reciprocal's error moves x
-  // by less than 2^-20
+  // per 2^-20 of a row. The reciprocal (one unit in the last place) and the
+  // two products move a cut of a piece of up to 16 px by up to 2^-18. Against
+  // the oracle in f64 the masks are nearer than the tile pipeline's, which
+  // rounds its records to f32: thirty triangles within 16 x 4 px 7.4e-7 of the mask's norm,
+  // 2.6e-6 there, sixty within 16 x 1 2.1e-6, 9.4e-6, text 2.5e-7 to 4.7e-7, 6.5e-7 to 1.2e-6.
   const float slope = Y1 > Y0 ? (x1 - x0) * __builtin_amdgcn_rcpf((float)(Y1 - Y0)) : 0.0f;
   for (int r = q.r0; r < q.r1; ++r) {
     const int ry = (r - q.r0) << rzg::kFixShift;

@@ -708,11 +708,17 @@ __device__ inline void scene_tile(const SceneFineArgs& a, TileLDS<kGroup>* Ls, u
 
 // Waves of a tile's workgroup. One wave takes a tile's paths one after the
 // other, which is the shortest time a frame can take however few tiles there
-// are; where the tiles leave the chip's 5,000 places for these waves idle
-// (five per SIMD, held there by their LDS), four waves share a tile's paths.
-// k_scene_fine of 240 shapes at 601x455 (1,102 tiles) 195 -> 176 us (what is
-// left is one tile with a path of thousands of records), of a tree of 49 fills
-// at 397x301 91 -> 64 us, of 16 paths at 256x256 30 -> 15 us.
+// are; four waves share them where the tiles are few. They pay for it with
+// their merge and three waves of a tile that has little in it, so that with
+// more tiles the crowded scenes still gain what the sparse ones lose. Whole
+// frames, one wave and four: at 256 tiles 2,000 circles 400, 201 us, 30 92, 87;
+// at 1,024 224, 159 and 88, 89; at 1,936 182, 163 and 87, 92 (50 gradients
+// over most of the view 313, 272); at 3,600 168, 169 and 88, 100. The line
+// lies where the sparse scenes lose about a twentieth. k_scene_fine of 240
+// shapes at 601x455 (1,102 tiles) 195 -> 176 us (what is left is one tile with
+// a path of thousands of records), of a tree of 49 fills at 397x301 91 -> 64
+// us, of 16 paths at 256x256 30 -> 15 us. The split changes the rounding of a
+// blend: the last bits of a pixel depend on which of the two its view took.
 constexpr int kSplit = 4;
 inline int scene_split(uint32_t n_tiles, uint32_t n_paths, uint32_t n_cus) {
   return n_tiles <= 8 * n_cus && n_paths >= 8 ? kSplit : 1;
@@ -724,12 +730,14 @@ inline int scene_split(uint32_t n_tiles, uint32_t n_paths, uint32_t n_cus) {
 // costliest first, until none is left: the tiles with the most paths start
 // first instead of last. The queue head comes as its own restrict parameter:
 // the compiler then knows its atomics touch nothing the tiles read.
-// MINW: waves per SIMD the registers must allow (1: no bound; 6: 96 VGPRs,
-// for the five waves that LDS holds; 8: 80 VGPRs with some spilled). LONG: the
+// BUDGET: RZ_PARAM_SCENE_WAVES, a register budget (1: no bound; 6: 96 VGPRs,
+// for the five waves per SIMD that LDS holds; 8: 80 VGPRs with some spilled,
+// for six waves of S = 1; the tiles of S = 4 do not fit six, and it bounds
+// nothing there). LONG: the
 // scene has a gradient that blend_gradient does not take (long_gradient).
 // S: waves of a tile.
-template <int MINW, bool QUEUE, bool LONG, int S>
-__global__ __launch_bounds__(64 * S, MINW == 6 ? 5 : MINW == 8 ? 6 : 1) void k_scene_fine(
+template <int BUDGET, bool QUEUE, bool LONG, int S>
+__global__ __launch_bounds__(64 * S, BUDGET == 6 ? 5 : BUDGET == 8 && S == 1 ? 6 : 1) void k_scene_fine(
     SceneFineArgs a, uint32_t* __restrict__ queue) {
   __shared__ TileLDS<kGroup> L[S];
   __shared__ uint32_t next;

@@ -117,6 +117,8 @@ def test_queued_tiles(waves, long):
         ctx.set_param(rz._abi.RZ_PARAM_SCENE_QUEUE, 1)
         for _ in range(3):
             assert np.array_equal(render(), ref), budget
+    ctx.set_param(rz._abi.RZ_PARAM_FINE_LDS, 32)  # four times as much for four waves
+    assert np.array_equal(render(), ref)
     ds.close()
     ctx.close()
 
