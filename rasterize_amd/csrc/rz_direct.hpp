@@ -1,7 +1,8 @@
 // Rasterizer::mask of a small path in one workgroup: flatten, signed-area
 // accumulation (src/rasterize.rs:365-470) and row sums with the whole mask in
 // LDS, without the binning stage. Used for the glyphs of an atlas whose masks
-// fit (direct_lds); larger ones go through the tile pipeline.
+// fit (direct_lds) where that takes a set less time than the tile pipeline
+// (DirectSet).
 #pragma once
 #include <algorithm>
 #include <cmath>
