@@ -210,6 +210,7 @@ def lines(n, w, h, k, seed=16):
     ("beyond the accumulators", lambda: of(3, 132, 137, 40), False),
     ("few long lines", lambda: lines(100, 100, 100, 30), True),
     ("many long lines", lambda: lines(100, 100, 100, 200), False),
+    ("many long lines in more glyphs", lambda: lines(400, 100, 100, 200), False),
     ("few segments in few glyphs", lambda: of(20, 64, 64, 100, "lq"), True),
     ("many segments in few glyphs", lambda: of(20, 64, 64, 900, "lq"), False),
     ("many segments in many glyphs", lambda: of(1500, 64, 64, 400, "lq"), True),
